@@ -355,6 +355,20 @@ template <int L> __device__ inline float group_sum(float v) {
   return v;
 }
 
+// Inclusive prefix sum over the 64 lanes of a wave in DPP: shifts by 1, 2, 4
+// and 8 lanes within each row of 16 (a lane with no source adds 0), then lane
+// 15's total broadcast to rows 1 and 3 and lane 31's to rows 2 and 3 (the GCN
+// wave scan of AMD's cross-lane operations guide).
+__device__ inline int wave_incl_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31
+  return v;
+}
+
 // Two-phase staging of nr activation rows (row r starts at row_of(r), K
 // halves each) into LDS in decode pair order with per-chunk sums:
 //   xs  [nr][4][C] uint4 (word jw of chunk c of row r at (r*4 + jw)*C + c),

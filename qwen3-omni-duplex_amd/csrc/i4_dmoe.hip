@@ -10,8 +10,9 @@
 // and down [E][H][I], either in the activation dtype or int8 with one scale per
 // output row (the q8 mode, fused_moe.py:84-94: value = q * scale).
 //
-// Decode-shaped: the T tokens of a call run in one launch per stage (grid z / y),
-// each token streaming its own experts' rows.
+// Decode-shaped, for calls of less than DG_MIN_T tokens (longer ones are grouped by
+// expert, i4_dmoe_group.hip): the T tokens of a call run in one launch per stage (grid
+// z / y), each token streaming its own experts' rows.
 //   k_d_gate_up  one workgroup per (block of rows of gate and up, slot, token);
 //                slot < topk is a routed expert, ranked from the logits by every
 //                wave itself (workgroup (0, 0, t) also stores token t's routing);
@@ -28,92 +29,12 @@
 // per word) and converted exactly to fp32; sum (q + 128) x - 128 sum x over
 // each 16-byte chunk uses the chunk sums staged with the activations, and the
 // row's scale multiplies the finished dot product once.
-#include "i4_common.h"
+#include "i4_dmoe.h"
+#include "i4_dmoe_group.h"
 #include "i4_launch.h"
 #include "i4_topk.h"
 
 namespace i4 {
-
-static constexpr int DWG = 256;   // threads per workgroup
-static constexpr int DMAXC = 8;   // 16-byte chunks of one weight row held per lane
-// polls of a single-launch down workgroup before it gives up (a launch whose
-// workgroups are dispatched in block order never reaches it)
-static constexpr int kHandPolls = 1 << 20;
-
-struct DW {                // one stacked weight [E][N][K]
-  const void* data;        // 16-bit values, or int8 when scale != NULL
-  const uint16_t* scale;   // [E][N] in the activation dtype, or NULL
-  int64_t es;              // elements per expert (N * K)
-  int N, K;
-};
-
-template <int XT> __device__ inline float round_to(float v) {
-  return Half<XT>::to_f32(Half<XT>::from_f32(v));
-}
-
-// 16 bytes at chunk c of row n of expert e (bpe bytes per element)
-__device__ inline u32x4 drow16(const DW& w, int e, int n, int c, int bpe) {
-  const char* row = (const char*)w.data + ((int64_t)e * w.es + (int64_t)n * w.K) * bpe;
-  return ldg16(row + 16 * (int64_t)c);
-}
-
-template <int XT> __device__ inline float dot16(u32x4 w, u32x4 x, float a) {
-  a = Half<XT>::dot2(w.x, x.x, a);
-  a = Half<XT>::dot2(w.y, x.y, a);
-  a = Half<XT>::dot2(w.z, x.z, a);
-  return Half<XT>::dot2(w.w, x.w, a);
-}
-
-// byte B of w as a float (v_cvt_f32_ubyteB)
-template <int B> __device__ inline float ubyte(u32 w) { return (float)((w >> (8 * B)) & 0xFFu); }
-
-// 16 int8 weights against xf[0..3] (the chunk's 16 activations), xsum their sum
-__device__ inline float dot_i8(u32x4 w, const f32x4* xf, float xsum, float a) {
-  const u32 v[4] = {w.x ^ 0x80808080u, w.y ^ 0x80808080u, w.z ^ 0x80808080u,
-                    w.w ^ 0x80808080u};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const f32x4 x = xf[i];
-    a += ubyte<0>(v[i]) * x.x;
-    a += ubyte<1>(v[i]) * x.y;
-    a += ubyte<2>(v[i]) * x.z;
-    a += ubyte<3>(v[i]) * x.w;
-  }
-  return a - 128.f * xsum;
-}
-
-// Activation staging in LDS, K values of a row (K % 16 == 0):
-//   xs   [K / 8]  u32x4  the raw halves (16-bit weights)
-//   xf   [K / 4]  f32x4  the values in fp32 (int8 weights only, F32)
-//   xsum [K / 16] float  the sum of each 16 values (F32)
-// One 8-value unit u per call; the lanes holding units u and u ^ 1 must run
-// the call together (the chunk sum pairs them with a lane swizzle).
-template <int XT, bool F32>
-__device__ inline void commit_unit(int u, u32x4 d, u32x4* xs, f32x4* xf, float* xsum) {
-  xs[u] = d;
-  if constexpr (F32) {
-    const u32 w[4] = {d.x, d.y, d.z, d.w};
-    float f[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      f[2 * i] = Half<XT>::to_f32((uint16_t)(w[i] & 0xFFFFu));
-      f[2 * i + 1] = Half<XT>::to_f32((uint16_t)(w[i] >> 16));
-    }
-    xf[2 * u] = f32x4{f[0], f[1], f[2], f[3]};
-    xf[2 * u + 1] = f32x4{f[4], f[5], f[6], f[7]};
-    const float s = ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
-    const float o = __builtin_bit_cast(
-        float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, s), 0x041F));  // lane ^ 1
-    if ((u & 1) == 0) xsum[u >> 1] = s + o;
-  }
-}
-
-// byte offsets of the staging arrays for K staged values, and their total
-__host__ __device__ inline size_t stage_xf_off(int K) { return (size_t)K * 2; }
-__host__ __device__ inline size_t stage_xsum_off(int K) { return (size_t)K * 6; }
-__host__ __device__ inline size_t stage_bytes(int K, bool f32) {
-  return f32 ? (size_t)K * 6 + (size_t)K / 4 : (size_t)K * 2;
-}
 
 struct DGateUpArgs {
   const uint16_t* x;        // [T][H]
@@ -226,24 +147,6 @@ __device__ inline void gate_up_rows(const DGateUpArgs& a, const DW w, int e, uin
       st_coherent(dst + n0 + threadIdx.x, s_act[threadIdx.x]);
     }
   }
-}
-
-// sigmoid(g_s . x) of token row xr (H values), the dot product and the sigmoid
-// each rounded to the activation dtype as the reference's 16-bit Linear and
-// sigmoid round them (fused_moe.py:139); 1 without a gate.  Every thread of
-// the workgroup calls it and receives the value.
-template <int XT>
-__device__ inline float shared_gate_value(const uint16_t* sgate_w, const uint16_t* xr, int H) {
-  __shared__ float s_d[DWG / 64];
-  if (!sgate_w) return 1.f;
-  float d = 0.f;
-  for (int k = threadIdx.x; k < H; k += DWG)
-    d += Half<XT>::to_f32(sgate_w[k]) * Half<XT>::to_f32(xr[k]);
-  d = group_sum<64>(d);
-  if ((threadIdx.x & 63) == 0) s_d[threadIdx.x >> 6] = d;
-  __syncthreads();
-  const float z = round_to<XT>((s_d[0] + s_d[1]) + (s_d[2] + s_d[3]));
-  return round_to<XT>(1.f / (1.f + expf(-z)));
 }
 
 // grid (row blocks, topk + 1, T); RI8 / SI8: routed / shared weights are int8
@@ -470,8 +373,18 @@ namespace {
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+constexpr int DMAX_H = 2048;  // hidden sizes served
+// Tokens from which a call runs grouped by expert (i4_dmoe_group.hip).  The grouped path
+// is six launches instead of three, which an eager caller pays on the host: 42-44 us a
+// call up to 16 tokens, against 32 us (up to 8 tokens), 44.4 (12) and 56 (16) per token
+// (bf16; int8 the same).  Above: 117 -> 67 us at 37 tokens, 417 -> 95 at 150, 1832 -> 231
+// at 700; int8 121 -> 59, 458 -> 105, 2051 -> 307.
+constexpr int DG_MIN_T = 12;
+
 struct DmoeWs {
-  size_t logits, sel, wts, sg, status, act, act_s, total;
+  size_t logits, sel, wts, sg, status, act, act_s;
+  size_t perm, entries, n_entries, ys, ys_s;  // the grouped path (T >= DG_MIN_T)
+  size_t total;
 };
 
 // act_s follows act directly: the router launch of a single-launch decode
@@ -486,6 +399,16 @@ DmoeWs dmoe_ws_layout(int T, int E, int topk, int I, int Is) {
   l.status = o; o += align256(4);
   l.act = o;    o += align256((size_t)T * topk * I * 2);
   l.act_s = o;  o += align256((size_t)T * Is * 2);
+  l.perm = l.entries = l.n_entries = l.ys = l.ys_s = o;
+  if (T >= DG_MIN_T) {
+    const int Tc = T < DG_CHUNK ? T : DG_CHUNK;
+    l.perm = o;      o += align256((size_t)Tc * topk * 4);
+    l.entries = o;   o += align256(dg_max_entries(Tc, E, topk) * sizeof(int4));
+    l.n_entries = o; o += align256(4);
+    // fp32 slot outputs; the hidden size is not known here, so its limit
+    l.ys = o;        o += align256((size_t)Tc * topk * DMAX_H * 4);
+    l.ys_s = o;      o += align256(Is ? (size_t)Tc * DMAX_H * 4 : 0);
+  }
   l.total = o;
   return l;
 }
@@ -559,7 +482,7 @@ int dmoe_impl(const void* x, int x_dtype, int T, const i4_dmoe_weights* wts, int
   const i4_dweight& dn = wts->down;
   const int E = gu.E, I = gu.N / 2, H = gu.K;
   const bool has_shared = wts->shared_gate_up.data != nullptr;
-  if (T < 1 || T > 65535 || E < 1 || E > 512 || H < 16 || H > 2048 || H % 16 || I < 16 ||
+  if (T < 1 || T > 65535 || E < 1 || E > 512 || H < 16 || H > DMAX_H || H % 16 || I < 16 ||
       I % 16 || gu.N != 2 * I || topk < 1 || topk > E || topk > (has_shared ? 7 : 8))
     return I4_ERR_SHAPE;
   int rc = check_dweight(gu, E, 2 * I, H);
@@ -638,6 +561,35 @@ int dmoe_impl(const void* x, int x_dtype, int T, const i4_dmoe_weights* wts, int
   da.sdn = has_shared ? to_dw(wts->shared_down) : DW{nullptr, nullptr, 0, 0, 0};
   da.residual = (const uint16_t*)residual;
   da.out = (uint16_t*)out;
+  if (T >= DG_MIN_T && dg_formats(ri8, si8)) {
+    rc = i4_launch_topk(lg, x_dtype, T, E, topk, renorm, ga.sel, ga.wts, nullptr, 0, stream);
+    for (int t0 = 0; rc == I4_OK && t0 < T; t0 += DG_CHUNK) {
+      DGCall c;
+      c.x = ga.x + (size_t)t0 * H;
+      c.T = T - t0 < DG_CHUNK ? T - t0 : DG_CHUNK;
+      c.topk = topk;
+      c.E = E;
+      c.sel = ga.sel + (size_t)t0 * topk;
+      c.wts = ga.wts + (size_t)t0 * topk;
+      c.gu = ga.gu;
+      c.dn = da.dn;
+      c.sgu = ga.sgu;
+      c.sdn = da.sdn;
+      c.sgate_w = ga.sgate_w;
+      c.residual = da.residual ? da.residual + (size_t)t0 * H : nullptr;
+      c.out = da.out + (size_t)t0 * H;
+      c.perm = (int32_t*)(ws + l.perm);
+      c.entries = (int4*)(ws + l.entries);
+      c.n_entries = (int*)(ws + l.n_entries);
+      c.act = ga.act;
+      c.act_s = ga.act_s;
+      c.ys = (float*)(ws + l.ys);
+      c.ys_s = (float*)(ws + l.ys_s);
+      c.status = status;
+      rc = i4_launch_dg(c, x_dtype, stream);
+    }
+    return rc;
+  }
   const DHand hand{(const uint16_t*)lg, E, renorm, (const uint16_t*)x, ga.sgate_w,
                    down_wait ? max_polls : kHandPolls, status};
   const DHand* hp = one || down_wait ? &hand : nullptr;

@@ -74,21 +74,6 @@ __global__ __launch_bounds__(WG) void k_moe_combine(const uint16_t* __restrict__
 // and thread e owns expert e for the three exclusive prefix sums (tokens,
 // first-list entries, second-list entries), done as wave scans plus a sum of
 // the totals of the waves before its own.
-//
-// Inclusive prefix sum over the 64 lanes of a wave in DPP: shifts by 1, 2, 4
-// and 8 lanes within each row of 16 (a lane with no source adds 0), then lane
-// 15's total broadcast to rows 1 and 3 and lane 31's to rows 2 and 3 (the GCN
-// wave scan of AMD's cross-lane operations guide).
-__device__ inline int wave_incl_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);   // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);   // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);   // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31
-  return v;
-}
-
 // One pass over a thread's (token, slot) pairs, SPT of them loaded before any
 // is used (a loop that loads and uses one pair per turn waits a whole memory
 // round trip per pair).  f(s, e) runs for every pair s < ns with its expert e.

@@ -942,7 +942,9 @@ def dmoe_forward(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top
     per-output-row scales in the activation dtype.  Three launches (router
     logits, gate_up + SiLU + routing, down + combine); one token with router_w and 16-bit
     experts runs in two (router logits; gate_up and down in one launch, the down
-    workgroups waiting for the activations: dmoe_status reports a wait that gave up)."""
+    workgroups waiting for the activations: dmoe_status reports a wait that gave up);
+    12 tokens or more are grouped by expert, so that an expert's weights are read once
+    for all of its tokens (six launches), with the same result bit for bit."""
     dev = _lib.require_device(x, gate_up, down, router_w, logits, shared_gate_up, shared_down,
                               shared_gate_w, residual)
     xt = _lib.half_code(x.dtype)

@@ -342,3 +342,57 @@ def test_dmoe_tokens_are_independent(pkg, dev, T, q8):
         one = pkg.dmoe_forward(x[t:t + 1].contiguous(), gu, dn, K, **kw)
         assert torch.equal(out[t:t + 1], one), f"token {t} of {T}"
     assert torch.isfinite(out.float()).all()
+
+
+@pytest.mark.parametrize("T,case", [
+    (12, dict()), (13, dict(q8=True)),                      # the smallest grouped calls
+    (65, dict(skew=True)), (129, dict(skew=True, q8=True)),  # an expert of 64 tokens and more
+    (1030, dict()),                                          # two passes over the tokens
+    (40, dict(H=256, E=16, I=48, Is=32)), (40, dict(H=256, E=16, I=48, Is=32, q8=True)),
+    (33, dict(H=2048, E=8, I=1024, Is=1024)),                # the longest rows
+    (33, dict(H=2048, E=8, I=2048, Is=2048, q8=True, shared_q8=True)),
+    (33, dict(H=528, E=20, I=272, Is=528, fp16=True)),       # rows that end inside a lane round
+    (33, dict(H=528, E=20, I=272, Is=528, q8=True, shared_q8=True)),
+    (20, dict(shared=False, top_k=8, residual=True)),
+    (20, dict(shared_q8=True)),                              # served by the per-token kernels
+])
+def test_dmoe_grouped_equals_per_token(pkg, dev, T, case):
+    """Calls grouped by expert give the per-token kernels' output (calls of at most 8
+    tokens) bit for bit: entry and tile edges, every format, odd and extreme row lengths."""
+    case = dict(case)
+    shapes = {k: case.pop(k) for k in ("H", "E", "I", "Is") if k in case}
+    dt = torch.float16 if case.pop("fp16", False) else torch.bfloat16
+    h, top_k = shapes.get("H", H), case.get("top_k", 4 if "E" in shapes else K)
+    print(f"dmoe grouped T={T} {shapes} {case}", flush=True)
+    S = _stacks(dev, dt, seed=30 + T, **shapes)
+    g = torch.Generator(device=dev).manual_seed(31)
+    x = torch.randn(T, h, generator=g, device=dev).to(dt)
+    rw = S["rw"].clone()
+    if case.get("skew"):  # every token selects expert 3
+        x[:, 0] = 8.0
+        rw[3, 0] = 4.0
+    kw = dict(router_w=rw)
+    gu, dn = S["gu"], S["dn"]
+    if case.get("q8"):
+        gu, kw["gate_up_scale"] = pkg.quantize_q8(gu)
+        dn, kw["down_scale"] = pkg.quantize_q8(dn)
+    if case.get("shared", True):
+        kw.update(shared_gate_up=S["sgu"], shared_down=S["sdn"], shared_gate_w=S["sgw"])
+        if case.get("shared_q8"):
+            kw["shared_gate_up"], kw["shared_gate_up_scale"] = pkg.quantize_q8(S["sgu"])
+            kw["shared_down"], kw["shared_down_scale"] = pkg.quantize_q8(S["sdn"])
+    res = torch.randn(T, h, generator=g, device=dev).to(dt) if case.get("residual") else None
+
+    def call(a, b):
+        return pkg.dmoe_forward(x[a:b].contiguous(), gu, dn, top_k, return_routing=True,
+                                residual=None if res is None else res[a:b].contiguous(), **kw)
+
+    got = call(0, T)
+    assert torch.isfinite(got[0].float()).all()
+    if case.get("skew"):
+        assert (got[1] == 3).sum() == T
+    for a in range(0, T, 8):
+        if T > 200 and 16 <= a < T - 24 and a % 128:
+            continue
+        for u, v in zip(got, call(a, min(a + 8, T))):
+            assert torch.equal(u[a:a + 8], v), f"tokens {a}.. of {T}"
