@@ -22,7 +22,7 @@ ARCH = os.environ.get("I4_OFFLOAD_ARCH", "gfx950")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
-    f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
+    f"--offload-arch={ARCH}", "-O3", "-std=c++20", "-fPIC",
     # packed fp32 VALU forms are kept out of the device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I", str(INCLUDE), "-I", str(CSRC),
@@ -32,7 +32,8 @@ FLAGS = [
 
 # per-source flags: the MFMA kernels keep their accumulators in VGPRs (the
 # group corrections read them every superchunk; AGPRs would need a move each way)
-EXTRA = {"i4_moe_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+         for f in ("i4_moe_mfma.hip", "i4_tile_gemm.hip", "i4_awq_mm.hip")}
 
 
 def sources() -> list[Path]:

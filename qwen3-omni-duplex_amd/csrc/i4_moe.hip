@@ -29,6 +29,7 @@ namespace i4 {
 
 static constexpr int WG = 256;
 static constexpr int TCHUNK = 1024;  // tokens handled by one pass of the pipeline
+static constexpr int BIG_CHUNK = 4096;  // and by one of the passes on 128-token tiles
 
 // out[t] = residual[t] + sum_j w[t][j] ys[t][j] in slot order, ys [T * topk][H]
 // in the activation dtype (each expert's output rounded as the reference rounds
@@ -198,7 +199,71 @@ __global__ __launch_bounds__(1024) void k_group(const int32_t* __restrict__ sel,
              n_mf_entries, lds);
 }
 
-
+// The grouping for the tiles of i4_tile_gemm.hip: one workgroup per expert, so its time
+// does not grow with what one workgroup can hold (k_group at T = 1024: 11 us).  Workgroup e
+// reads every pair once, in order: the pairs of lower experts give its first position, its
+// own pairs wait in LDS in pair order.  Entry q of expert e goes to slot
+// off / TG_TOK + e + q, which no other expert uses (the next expert's first slot is at
+// least ceil(c / TG_TOK) further); slots left free hold an empty entry.  There are
+// T topk / TG_TOK + E slots.
+__global__ __launch_bounds__(1024) void k_group_e(const int32_t* __restrict__ sel, int ns, int E,
+                                                  int32_t* __restrict__ perm,
+                                                  int4* __restrict__ entries,
+                                                  int* __restrict__ n_entries,
+                                                  int32_t* __restrict__ status) {
+  __shared__ int s_id[BIG_CHUNK];
+  __shared__ int s_c[2][16], s_lo[16];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, me = blockIdx.x;
+  if (me == 0 && tid == 0) {
+    if (status) *status = I4_OK;
+    *n_entries = ns / TG_TOK + E;
+  }
+  const uint64_t below = (1ull << lane) - 1;
+  int c = 0, lo = 0;
+  for (int s0 = 0, it = 0; s0 < ns; s0 += 4096, it ^= 1) {
+    int e[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) e[u] = sel[min(s0 + 4 * tid + u, ns - 1)];
+    int mine = 0, rank = 0, total = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const bool in = s0 + 4 * tid + u < ns;
+      const uint64_t m = __ballot(in && e[u] == me);
+      rank += __popcll(m & below);
+      total += __popcll(m);
+      mine |= (int)(in && e[u] == me) << u;
+      lo += in && (unsigned)e[u] < (unsigned)me;
+    }
+    if (lane == 0) s_c[it][wave] = total;
+    __syncthreads();
+    int base = c;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const int v = s_c[it][w];
+      base += w < wave ? v : 0;
+      c += v;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if ((mine >> u) & 1) {
+        const int at = base + rank++;
+        if (at < BIG_CHUNK) s_id[at] = s0 + 4 * tid + u;
+      }
+  }
+  lo = (int)group_sum<64>((float)lo);  // exact: fewer than 2^24 pairs
+  if (lane == 0) s_lo[wave] = lo;
+  __syncthreads();
+  int off = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) off += s_lo[w];
+  c = min(c, BIG_CHUNK);
+  for (int i = tid; i < c; i += 1024) perm[off + i] = s_id[i];
+  const int s_first = off / TG_TOK + me;
+  const int s_end = me == E - 1 ? ns / TG_TOK + E : (off + c) / TG_TOK + me + 1;
+  for (int q = tid; q < s_end - s_first; q += 1024)
+    entries[s_first + q] =
+        int4{me, off + q * TG_TOK, max(0, min(TG_TOK, c - q * TG_TOK)), 0};
+}
 
 }  // namespace i4
 
@@ -209,6 +274,18 @@ using namespace i4;
 namespace {
 
 inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Whether a pass of more than TCHUNK tokens takes the 128-token tiles: whole column tiles,
+// and 64 tokens per expert on average.  Both sides, us per block of 128 experts (top-8, H
+// 2048, I 768), 64-token tiles in passes of at most 1024 tokens / 128-token tiles: bf16
+// groups of 32: 1000 tokens 271 / 290, 1500 about 390 / 362, 2400 about 620 / 478; fp16
+// groups of 128: 210 / 232, 345 / 296, 538 / 415.
+inline bool tile_gemm_fits(int H, int I, int E, int topk) {
+  return I % (16 * TG_NW) == 0 && H % (32 * TG_NW) == 0 && TCHUNK * topk >= 64 * E;
+}
+inline int tokens_per_pass(int H, int I, int E, int topk) {
+  return tile_gemm_fits(H, I, E, topk) ? BIG_CHUNK : TCHUNK;
+}
 
 struct MoeWs {
   void* logits;
@@ -228,7 +305,7 @@ struct MoeWs {
 };
 
 MoeWs carve(void* base, int T, int H, int I, int E, int topk) {
-  const int Tc = T < TCHUNK ? T : TCHUNK;
+  const int tc = tokens_per_pass(H, I, E, topk), Tc = T < tc ? T : tc;
   const size_t Tk = (size_t)Tc * topk;
   MoeWs m;
   size_t o = 0;
@@ -291,6 +368,8 @@ struct MoeOps {
                     hipStream_t);
   int (*mfma_gd)(int, const void*, int, int, const int4*, const int*, const int32_t*, const TW&,
                  const TW&, int, void*, void*, int32_t*, int, bool, hipStream_t);
+  int (*tile_gemm)(bool, int, const void*, int, int, const int4*, const int*, const int32_t*,
+                   const TW&, int, void*, hipStream_t);
 };
 
 template <int XT, int ST> constexpr MoeOps moe_ops() {
@@ -298,7 +377,8 @@ template <int XT, int ST> constexpr MoeOps moe_ops() {
                 &launch_gate_up_ct<XT, ST>,  &launch_down_m1_ct<XT, ST>,
                 &launch_mfma_gate_up<XT, ST>, &launch_mfma_down<XT, ST>,
                 &launch_moe_m1_ct<XT, ST>,   &launch_mfma_mixed<XT, ST>,
-                &launch_moe_m1x_ct<XT, ST>,  &launch_mfma_gd<XT, ST>};
+                &launch_moe_m1x_ct<XT, ST>,  &launch_mfma_gd<XT, ST>,
+                &launch_tile_gemm_moe<XT, ST>};
 }
 
 bool pick_ops(int xt, int gst, int dst, MoeOps* ops) {
@@ -439,6 +519,7 @@ int moe_chunk(const void* x, int xt, int T, const i4_moe_weights* mw, const i4_q
     lg = ws.logits;
     if (mw->norm_w) x = ws.xn;
   }
+  const bool big = T > TCHUNK;  // only passes on the 128-token tiles hold so many
   const int TW_ = (T + 31) / 32;
   const size_t glds = (size_t)2 * E * TW_ * 4 + (size_t)E * 4;
   // T <= MF_TOK: no expert has more tokens than one large entry holds, and
@@ -451,9 +532,13 @@ int moe_chunk(const void* x, int xt, int T, const i4_moe_weights* mw, const i4_q
     rc = i4_launch_topk(lg, xt, T, E, topk, renorm, sel, wts, nullptr, 0, s, pend, n_pend);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(k_group, dim3(1), dim3(1024), glds, s, sel, T, topk, E,
-                     one_list ? T : MF_SMALL, MF_SMALL, ws.perm, ws.entries, ws.n_entries,
-                     ws.mf_entries, ws.n_mf_entries, st_reset, fused ? ws.epoch : nullptr);
+  if (big)
+    hipLaunchKernelGGL(k_group_e, dim3(E), dim3(1024), 0, s, sel, Tk, E, ws.perm, ws.entries,
+                       ws.n_entries, st_reset);
+  else
+    hipLaunchKernelGGL(k_group, dim3(1), dim3(1024), glds, s, sel, T, topk, E,
+                       one_list ? T : MF_SMALL, MF_SMALL, ws.perm, ws.entries, ws.n_entries,
+                       ws.mf_entries, ws.n_mf_entries, st_reset, fused ? ws.epoch : nullptr);
   if (hipGetLastError() != hipSuccess) return I4_ERR_LAUNCH;
   // entry counts: sum over experts of ceil(n_e / 16) <= min(E, Tk) + Tk / 16
   const int max_s = (E < Tk ? E : Tk) + (one_list ? Tk / MF_SMALL : 0);
@@ -467,6 +552,14 @@ int moe_chunk(const void* x, int xt, int T, const i4_moe_weights* mw, const i4_q
                           ws.act, s);
     if (rc) return rc;
     rc = ops.mfma_down(true, max_s, ws.act, Tk, ws.entries, ws.n_entries, ws.perm, tdn, ws.ys, s);
+    if (rc) return rc;
+  } else if (big) {
+    const int max_e = E + Tk / TG_TOK;
+    rc = ops.tile_gemm(true, max_e, x, T, topk, ws.entries, ws.n_entries, ws.perm, tgu, I, ws.act,
+                       s);
+    if (rc) return rc;
+    rc = ops.tile_gemm(false, max_e, ws.act, Tk, topk, ws.entries, ws.n_entries, ws.perm, tdn, I,
+                       ws.ys, s);
     if (rc) return rc;
   } else {  // large and small entries of a projection share one launch
     rc = ops.mfma_mixed(true, max_b, max_s, x, T, topk, ws.mf_entries, ws.n_mf_entries,
@@ -514,8 +607,9 @@ int moe_forward_impl(const void* x, int x_dtype, int T, const i4_moe_weights* we
   if ((uintptr_t)workspace & 255) return I4_ERR_ALIGN;
   MoeWs ws = carve(workspace, T, H, I, E, topk);
   if (status) ws.status = status;  // the caller's status word instead of the workspace's
-  for (int t0 = 0; t0 < T; t0 += TCHUNK) {
-    const int Tc = T - t0 < TCHUNK ? T - t0 : TCHUNK;
+  const int tc = tokens_per_pass(H, I, E, topk);
+  for (int t0 = 0; t0 < T; t0 += tc) {
+    const int Tc = T - t0 < tc ? T - t0 : tc;
     const char* xs = (const char*)x + (size_t)t0 * H * 2;
     const void* lg = logits ? (const char*)logits + (size_t)t0 * E * 2 : nullptr;
     const void* rs = residual ? (const char*)residual + (size_t)t0 * H * 2 : nullptr;

@@ -13,6 +13,8 @@ static constexpr int MF_TOK = 64;    // tokens per entry of the large-entry MFMA
 static constexpr int LIN_TOK = 64;   // rows per tile of the dense linear MFMA launch
 static constexpr int ONE_LIST_T = 64;  // up to this many tokens: small entries only
 static constexpr int MF_SMALL = 16;  // experts with at most this many tokens: one m-block
+static constexpr int TG_TOK = 128;   // rows per tile of i4_tile_gemm.hip
+static constexpr int TG_NW = 8;      // its waves (32 weight rows each)
 static constexpr int MF_NB = 2;      // n-blocks of 16 weight rows per wave
 
 // decode gate_up + SiLU: slot j of token 0 (route: ranked from logits in the
@@ -134,5 +136,26 @@ template <int XT, int ST>
 int launch_mfma_linear(const void* x, int M, const TW& w, const void* bias, void* y, int ot,
                        void* ws, size_t ws_bytes, hipStream_t s);
 size_t linear_tile_workspace_bytes(int M, int N, int K);
+// y = the sum of ksplit fp32 partials [ksplit][M][N] in order (+ bias), in dtype ot
+int launch_linear_finish(const float* part, int ksplit, int M, int N, const void* bias, void* y,
+                         int ot, hipStream_t s);
+
+// Dense linear layer on AutoAWQ weights in place (i4_awq_mm.hip), E = 1, N % 8 == 0; part:
+// awq_mm_ksplit() x M x N fp32 (unused when that is 1).
+int awq_mm_ksplit(int M, int N, int K);
+bool awq_mm_fits(int M, int N, int K);
+template <int XT, int ST>
+int launch_awq_mm(const void* x, int M, const i4_qweight& w, const void* bias, void* y, int ot,
+                  float* part, hipStream_t s);
+
+// The same projections in tiles of TG_TOK rows x 32 TG_NW weight rows (i4_tile_gemm.hip):
+// entries of <= TG_TOK tokens; I % (16 TG_NW) == 0 and N % (32 TG_NW) == 0.
+template <int XT, int ST>
+int launch_tile_gemm_linear(const void* x, int M, const TW& w, const void* bias, void* y, int ot,
+                            hipStream_t s);
+template <int XT, int ST>
+int launch_tile_gemm_moe(bool gate_up, int max_entries, const void* src, int src_rows, int topk,
+                         const int4* ent, const int* nent, const int32_t* perm, const TW& w,
+                         int I, void* out, hipStream_t s);
 
 }  // namespace i4

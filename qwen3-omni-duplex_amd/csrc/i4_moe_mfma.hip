@@ -16,9 +16,14 @@
 //         <= 2^-11, the numerics of dequantise-then-multiply) and the MFMA
 //         accumulates straight into the result: no second accumulator, which
 //         keeps a 64-token entry within 128 VGPRs.
-//   bf16: B holds M + q exactly (gfx950 has no packed bf16 add or multiply)
-//         and a group ends with res += s D - s (M + z) S_m, S_m the sum of
-//         token m's activations over the group.
+//   bf16: B holds M + q exactly (gfx950 has no packed bf16 add or multiply),
+//         the accumulator starts at -(M + z) S_m, S_m the sum of token m's
+//         activations over the group, and a group ends with res += s D.  S_m is
+//         staged with the activations, four tokens to one 16-byte read, and
+//         scaled by -(M + 8) there when the weight has no zero points.  (The
+//         correction after the products, eight fp32 operations per MFMA and four
+//         4-byte LDS reads per m-block, took the 1500-row 2048 -> 5120 linear
+//         109 us; this form 93 us.)
 // Accumulation is fp32; apart from the fold every product is exact.
 //
 // All global reads are raw buffer loads: one descriptor per operand (an
@@ -45,180 +50,9 @@
 //   DOWN:   NB blocks of output rows per wave, ys[slot] rounded to the
 //           activation dtype (the reference's y.to(x.dtype), fused_packed_moe.py:262); 64 NB rows
 //           per workgroup.
-#include "i4_moe_launch.h"
+#include "i4_tile_mfma.h"
 
 namespace i4 {
-
-// Staged activations: token m's 16 words of a superchunk are one 256-byte row, word w
-// at slot w ^ (m & 15) (xs_at).  An MFMA operand load (lanes = 16 tokens x 4
-// words) and a staging store (16 lanes = 4 tokens x 4 words) each touch every bank
-// once per 16 lanes; measured on gfx950, the swizzled rows read at 4.4 cycles per
-// wave-wide 16-byte load against 8.1 with a one-word pad per row.
-static constexpr int MF_TSTRIDE = 16;  // uint4 per staged token row
-__device__ inline int xs_at(int m, int w) { return m * MF_TSTRIDE + (w ^ (m & 15)); }
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-__device__ inline u32x4 bload16(rsrc_t r, u32 voff, int soff) {
-  return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-}
-// the same past the L1 (sc1): sees what other CUs of the launch wrote through
-__device__ inline u32x4 bload16_coherent(rsrc_t r, u32 voff, int soff) {
-  return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kCoherent);
-}
-__device__ inline u32 bload4(rsrc_t r, u32 voff, int soff) {
-  return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-}
-template <int ST> __device__ inline u32 bload_scale(rsrc_t r, u32 voff, int soff) {
-  if constexpr (ST == I4_F32) return __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-  else return (u32)__builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0);
-}
-
-template <int XT> __device__ inline f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-  if constexpr (XT == I4_F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
-                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-// 8 exact halves M + q of one tile word (nibble slots (p, p + 4) -> half pair p),
-// columns 8m .. 8m + 7 in order
-template <int XT> __device__ inline u32x4 decode8(u32 w, u32 mg) {
-  constexpr u32 MK = 0x000F000Fu;
-  return u32x4{(w & MK) | mg, ((w >> 4) & MK) | mg, ((w >> 8) & MK) | mg, ((w >> 12) & MK) | mg};
-}
-
-// fp16 pair (M + q0, M + q1) + nz, nz = (-(M + z), -(M + z)): exactly (q0 - z, q1 - z)
-__device__ inline u32 sub_zero(u32 p, u32 nz) {
-  return __builtin_bit_cast(u32, __builtin_bit_cast(f16x2, p) + __builtin_bit_cast(f16x2, nz));
-}
-
-// -(M + z) twice, fp16, for the zero point of group g held in zero word zw
-__device__ inline u32 neg_zero2(u32 zw, int g) {
-  return (0xE400u | ((zw >> (4 * (g & 7))) & 15u)) * 0x00010001u;
-}
-
-// B operand of one MFMA step (nz: neg_zero2 of the step's group, fp16 only;
-// mg: magic_v<XT>())
-template <int XT> __device__ inline u32x4 b_operand(u32 word, u32 nz, u32 mg) {
-  u32x4 b = decode8<XT>(word, mg);
-  if constexpr (XT == I4_F16) {
-    b.x = sub_zero(b.x, nz);
-    b.y = sub_zero(b.y, nz);
-    b.z = sub_zero(b.z, nz);
-    b.w = sub_zero(b.w, nz);
-  }
-  return b;
-}
-
-// the group scale as two fp16 copies (rounded to fp16 when stored wider)
-template <int ST> __device__ inline u32 scale_h2(u32 raw) {
-  if constexpr (ST == I4_F16) {
-    return (raw & 0xFFFFu) * 0x00010001u;
-  } else {
-    const u32 h = __builtin_bit_cast(uint16_t, (_Float16)scale_from_raw<ST>(raw));
-    return h * 0x00010001u;
-  }
-}
-
-// fp16 pairs a * s (one v_pk_mul_f16)
-__device__ inline u32 mul_h2(u32 a, u32 s) {
-  return __builtin_bit_cast(u32, __builtin_bit_cast(f16x2, a) * __builtin_bit_cast(f16x2, s));
-}
-
-// fp16 B operand times the group scale: (q - z) s, one rounding per element.
-// The components go through scalars: a bit cast applied directly to a vector
-// component expression (b.y) reads component 0 with this compiler.
-__device__ inline u32x4 scale_b(u32x4 b, u32 s2) {
-  const u32 b0 = b.x, b1 = b.y, b2 = b.z, b3 = b.w;
-  return u32x4{mul_h2(b0, s2), mul_h2(b1, s2), mul_h2(b2, s2), mul_h2(b3, s2)};
-}
-
-// first row block of n-block nb of wave `wave` in column tile `tile`
-template <bool GATEUP, int NB>
-__device__ inline int nblock(int tile, int wave, int nb, int I) {
-  if constexpr (GATEUP)
-    return tile * (2 * NB) + (NB / 2) * wave + (nb % (NB / 2)) + (nb >= NB / 2 ? (I >> 4) : 0);
-  else
-    return tile * (4 * NB) + NB * wave + nb;
-}
-
-// the weight operands of one wave: NB n-blocks of expert e, lane (r, j).
-// Lane offsets live in VGPRs; the n-block offsets are wave-uniform and go in
-// the scalar offset of each load, with the superchunk / group offset.
-template <int ST, int NB> struct WBuf {
-  rsrc_t p, s, z;
-  u32 lw, ls, lz;              // per-lane byte offsets
-  int bw[NB], bs[NB], bz[NB];  // per-n-block byte offsets (wave-uniform)
-  u32 zor;                     // 0x88888888 when the weight has no zero points
-  int gshift;
-};
-
-template <int ST, int NB>
-__device__ inline WBuf<ST, NB> wbuf(const TW& w, int e, const int (&blk)[NB], int r, int j) {
-  constexpr int SB = ST == I4_F32 ? 4 : 2;
-  const int SC = w.K >> 7;
-  const int NG = (w.K + (32 << w.gshift) - 1) >> (w.gshift + 5), NZW = (NG + 7) >> 3;
-  WBuf<ST, NB> b;
-  b.p = rsrc(w.packed + e * w.pes, (u32)w.N * (u32)(w.K >> 1));
-  b.s = rsrc((const char*)w.scale + e * w.ses * SB, (u32)w.N * NG * SB);
-  if (w.zeros) {
-    b.z = rsrc(w.zeros + e * w.zes, (u32)w.N * NZW * 4u);
-    b.zor = 0u;
-  } else {
-    b.z = rsrc(w.packed, 0u);
-    b.zor = 0x88888888u;
-  }
-  b.lw = (u32)r * 64u + (u32)j * 16u;
-  b.ls = (u32)r * SB;
-  b.lz = (u32)r * 4u;
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    b.bw[nb] = blk[nb] * SC * 1024;
-    b.bs[nb] = blk[nb] * NG * 16 * SB;
-    b.bz[nb] = blk[nb] * NZW * 64;
-  }
-  b.gshift = w.gshift;
-  return b;
-}
-
-// superchunk sc of every n-block: the 16-byte tile word, the raw scale(s) and
-// the zero word (one zero word covers the superchunk's groups).  Nothing here
-// touches the loaded values, so issuing never waits for a load.
-template <int ST, bool GB, int NB>
-__device__ inline void wissue(const WBuf<ST, NB>& b, int sc, TSlot<GB> (&o)[NB]) {
-  constexpr int SB = ST == I4_F32 ? 4 : 2;
-  const int g0 = (4 * sc) >> b.gshift;
-#pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    o[nb].w = bload16(b.p, b.lw, b.bw[nb] + sc * 1024);
-    if constexpr (GB) {
-      o[nb].s[0] = bload_scale<ST>(b.s, b.ls, b.bs[nb] + g0 * 16 * SB);
-    } else {
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        o[nb].s[t] = bload_scale<ST>(b.s, b.ls, b.bs[nb] + ((4 * sc + t) >> b.gshift) * 16 * SB);
-    }
-    o[nb].z = bload4(b.z, b.lz, b.bz[nb] + (g0 >> 3) * 64);  // | zor where it is used
-  }
-}
-
-// group correction of one n-block's accumulator (rows m = 4 j + i of column r)
-template <int XT, int ST>
-__device__ inline void correct(f32x4& res, const f32x4& d, u32 sraw, u32 zw, int g,
-                               const float (&sm)[4]) {
-  const float sv = scale_from_raw<ST>(sraw);
-  if constexpr (XT == I4_F16) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) res[i] = fmaf(sv, d[i], res[i]);
-  } else {
-    const float bv = -sv * (Half<XT>::MAGIC + (float)((zw >> (4 * (g & 7))) & 15u));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) res[i] = fmaf(sv, d[i], fmaf(bv, sm[i], res[i]));
-  }
-}
 
 // One entry (<= 16 MB tokens of one expert) x one column tile.  MB m-blocks
 // of 16 tokens (1 for the small entries, 4 for the large ones), NB n-blocks
@@ -302,6 +136,8 @@ __device__ inline void tile_mfma_body(
     u32x4 x[XR ? WPT : 1];
   };
   u32x4 xd[WPT];
+  const bool sym = !w.zeros;  // every zero point 8
+  const float xscale = sym ? -(Half<XT>::MAGIC + 8.f) : -1.f;  // of the staged bf16 sums
   const rsrc_t hr = rsrc(HAND && !GATEUP ? hsrc : src, src_bytes);
   // HAND down reads act through the caches first (an entry's activations are read by
   // every column tile of it); only a word that still holds the pending pattern, in memory
@@ -340,12 +176,12 @@ __device__ inline void tile_mfma_body(
     if constexpr (!EXACT) {
       if constexpr (MB == 1) {
         sm = group_sum<4>(sm);  // the chunk's 4 words sit in 4 adjacent lanes
-        if ((kw & 3) == 0) XSUM(buf, 4 * tk + (kw >> 2)) = sm;
+        if ((kw & 3) == 0) XSUM(buf, TOK * (kw >> 2) + tk) = xscale * sm;
       } else if constexpr (MB == 4) {
-        XSUM(buf, 4 * tk + (kw >> 2)) = sm;
+        XSUM(buf, TOK * (kw >> 2) + tk) = xscale * sm;
       } else {  // two chunks per thread
-        XSUM(buf, 4 * tk + (kw >> 2)) = sm;
-        XSUM(buf, 4 * tk + (kw >> 2) + 1) = sm1;
+        XSUM(buf, TOK * (kw >> 2) + tk) = xscale * sm;
+        XSUM(buf, TOK * ((kw >> 2) + 1) + tk) = xscale * sm1;
       }
     }
   };
@@ -358,16 +194,13 @@ __device__ inline void tile_mfma_body(
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) res[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // S of rows 16 mb + 4 j + i over chunks [t0, t0 + nt) of the staged superchunk
-  auto rows_sum = [&](int buf, int mb, int t0, int nt, float (&sm)[4]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float* p = &XSUM(buf, 4 * (16 * mb + 4 * kb + i));
-      float v = 0.f;
-      for (int t = t0; t < t0 + nt; ++t) v += p[t];
-      sm[i] = v;
-    }
+  // bf16: the staged sums of rows 16 mb + 4 j .. + 3 over chunk t (one 16-byte read)
+  auto rows_sum = [&](int buf, int mb, int t) {
+    return *(const f32x4*)&XSUM(buf, TOK * t + 16 * mb + 4 * kb);
   };
+  // accumulator start of a group, bf16: -(M + z) S_m from the staged sums and mz, the M + z
+  // of the lane's column (1 for a weight without zero points: xscale holds it)
+  auto start = [](const f32x4& sm, float mz) { return sm * mz; };
   auto compute = [&](int sc, const TSlot<GB> (&sl)[NB], int buf) {
     const int g0 = (4 * sc) >> w.gshift;
     u32 zw[NB], nz[NB];  // zero words; GB: one zero point for the superchunk
@@ -410,63 +243,66 @@ __device__ inline void tile_mfma_body(
       }
       return;
     } else {
-    // exact: B = q - z (fp16) or M + q (bf16), per-group correction (bf16 with
-    // the activation sums)
+    // exact: B = q - z (fp16) or M + q (bf16); a group ends with res += s D
     f32x4 d[MB][NB];
+    float mz[NB];
+    if constexpr (GB) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+      for (int nb = 0; nb < NB; ++nb)
+        mz[nb] = EXACT ? 0.f : sym ? 1.f : Half<XT>::MAGIC + zero_of(zw[nb], g0);
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb) d[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int mb = 0; mb < MB; ++mb) {
+        if (mb < nmb) {
+          f32x4 sm = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (!EXACT)
+            sm = (rows_sum(buf, mb, 0) + rows_sum(buf, mb, 1)) +
+                 (rows_sum(buf, mb, 2) + rows_sum(buf, mb, 3));
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) d[mb][nb] = EXACT ? sm : start(sm, mz[nb]);
+        }
+      }
+    }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int g = (4 * sc + t) >> w.gshift;
-      if constexpr (MB == 1) {  // one m-block: each B operand feeds one MFMA
-        const u32x4 a = XS(buf, xs_at(ln, 4 * t + kb));
+      u32x4 b[NB];
+      auto bop = [&](int nb) {
+        return b_operand<XT>(word_t(sl[nb].w, t), GB ? nz[nb] : neg_zero2(zw[nb], g), mg);
+      };
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          d[0][nb] = mfma16<XT>(
-              a, b_operand<XT>(word_t(sl[nb].w, t), GB ? nz[nb] : neg_zero2(zw[nb], g), mg),
-              d[0][nb]);
-      } else {
-        u32x4 b[NB];
+      for (int nb = 0; nb < NB; ++nb) {
+        if constexpr (MB > 1) b[nb] = bop(nb);  // one m-block: each feeds one MFMA
+        if constexpr (!GB && !EXACT) mz[nb] = sym ? 1.f : Half<XT>::MAGIC + zero_of(zw[nb], g);
+      }
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          b[nb] = b_operand<XT>(word_t(sl[nb].w, t), GB ? nz[nb] : neg_zero2(zw[nb], g), mg);
+      for (int mb = 0; mb < MB; ++mb) {
+        if (mb < nmb) {
+          const u32x4 a = XS(buf, xs_at(16 * mb + ln, 4 * t + kb));
+          if constexpr (!GB) {
+            f32x4 sm = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (!EXACT) sm = rows_sum(buf, mb, t);
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          if (mb < nmb) {
-            const u32x4 a = XS(buf, xs_at(16 * mb + ln, 4 * t + kb));
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) d[mb][nb] = mfma16<XT>(a, b[nb], d[mb][nb]);
+            for (int nb = 0; nb < NB; ++nb) d[mb][nb] = EXACT ? sm : start(sm, mz[nb]);
           }
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            d[mb][nb] = mfma16<XT>(a, MB > 1 ? b[nb] : bop(nb), d[mb][nb]);
         }
       }
       if constexpr (!GB) {
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          if (mb < nmb) {
-            float sm[4] = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (!EXACT) rows_sum(buf, mb, t, 1, sm);
+        for (int mb = 0; mb < MB; ++mb)
+          if (mb < nmb)
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-              correct<XT, ST>(res[mb][nb], d[mb][nb], sl[nb].s[t], zw[nb], g, sm);
-              d[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-          }
-        }
+            for (int nb = 0; nb < NB; ++nb) add_group<ST>(res[mb][nb], d[mb][nb], sl[nb].s[t]);
       }
     }
     if constexpr (GB) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        if (mb < nmb) {
-          float sm[4] = {0.f, 0.f, 0.f, 0.f};
-          if constexpr (!EXACT) rows_sum(buf, mb, 0, 4, sm);
+      for (int mb = 0; mb < MB; ++mb)
+        if (mb < nmb)
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-            correct<XT, ST>(res[mb][nb], d[mb][nb], sl[nb].s[0], zw[nb], g0, sm);
-        }
-      }
+          for (int nb = 0; nb < NB; ++nb) add_group<ST>(res[mb][nb], d[mb][nb], sl[nb].s[0]);
     }
     }
   };
@@ -610,7 +446,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   constexpr int TOK = 16 * MB;
   constexpr int NBUF = MB <= 4 ? 2 : 1;  // 128-token tiles are staged single-buffered
   __shared__ u32x4 xs[NBUF][TOK * MF_TSTRIDE];
-  __shared__ float xsum[NBUF][TOK * 4];  // bf16: per token and chunk
+  __shared__ __align__(16) float xsum[NBUF][TOK * 4];  // bf16: per token and chunk
   // one-m-block entries alone: two ring slots keep the wave at <= 80 VGPRs, so six
   // workgroups fit a CU and the T <= 64 launches run in one round
   tile_mfma_body<XT, ST, GB, GATEUP, NB, MB, LIN, (MB == 1 && !LIN) ? 2 : 3>(
@@ -633,7 +469,7 @@ __global__ __launch_bounds__(256) void k_tile_mfma_mixed(
   constexpr int TOKL = MF_TOK;
   constexpr int NBUF = MF_TOK <= 64 ? 2 : 1;  // 128-token tiles are staged single-buffered
   __shared__ u32x4 xs[NBUF * TOKL * MF_TSTRIDE];
-  __shared__ float xsum[NBUF * TOKL * 4];
+  __shared__ __align__(16) float xsum[NBUF * TOKL * 4];
   const int y = blockIdx.y, nl = *n_large;
   if (y < nl)
     tile_mfma_body<XT, ST, GB, GATEUP, NB, MF_TOK / 16, false, 2>(
@@ -675,7 +511,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     uint16_t* act, u32 act_bytes, float* __restrict__ ys, int n_e, int gu_cols, int dn_cols,
     int down_only, int max_polls, int32_t* __restrict__ status) {
   __shared__ u32x4 xs[2 * 16 * MF_TSTRIDE];
-  __shared__ float xsum[2 * 16 * 4];
+  __shared__ __align__(16) float xsum[2 * 16 * 4];
   bool dn;
   int e, tile;
   gd_map((int)blockIdx.x, n_e, gu_cols, dn_cols, down_only, dn, e, tile);
@@ -807,6 +643,7 @@ __global__ __launch_bounds__(256) void k_linear_finish(const float* __restrict__
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
   float v = 0.f;
+#pragma unroll 4
   for (int z = 0; z < ksplit; ++z) v += part[z * total + i];
   const int n = (int)(i % N);
   if (ot == I4_F32) {
@@ -821,6 +658,14 @@ __global__ __launch_bounds__(256) void k_linear_finish(const float* __restrict__
   }
 }
 
+int launch_linear_finish(const float* part, int ksplit, int M, int N, const void* bias, void* y,
+                         int ot, hipStream_t s) {
+  const int64_t total = (int64_t)M * N;
+  hipLaunchKernelGGL(k_linear_finish, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
+                     part, ksplit, total, N, bias, y, ot);
+  return hipGetLastError() == hipSuccess ? I4_OK : I4_ERR_LAUNCH;
+}
+
 // K ranges of a dense linear launch: a grid of fewer than 256 output tiles
 // (few rows or few columns) is split along K until it has about 512
 // workgroups, each range keeping at least 4 superchunks
@@ -831,6 +676,18 @@ int linear_ksplit(int M, int N, int K) {
   int ks = (512 + tiles - 1) / tiles;
   if (ks > sc / 4) ks = sc / 4;
   return ks < 1 ? 1 : ks;
+}
+
+// Whether a dense linear launch takes the 128-row tiles: a round of 256 of them (one
+// workgroup per CU) takes the same time full or not, so they have to fill their rounds.
+// us, 64-row tiles / 128-row tiles at K 2048: bf16 groups of 32 at 112 tiles 44 / 50, 140
+// 67 / 52, 240 85 / 57, 320 119 / 100, 640 207 / 156; fp16 groups of 128 at 192 tiles
+// 40 / 41, 240 49 / 45, 320 63 / 77, 512 93 / 80, 640 113 / 117.
+static bool linear_big(int xt, int M, int N) {
+  if (N % (32 * TG_NW) != 0) return false;
+  const int64_t tiles = (int64_t)(N / (32 * TG_NW)) * ((M + TG_TOK - 1) / TG_TOK);
+  const int64_t slots = (tiles + 255) / 256 * 256;
+  return xt == I4_BF16 ? 2 * tiles > slots : 10 * tiles >= 9 * slots;
 }
 
 size_t linear_tile_workspace_bytes(int M, int N, int K) {
@@ -848,6 +705,7 @@ int launch_mfma_linear(const void* x, int M, const TW& w, const void* bias, void
     return I4_ERR_SHAPE;
   constexpr int COLS = 64 * MF_NB, TOK = LIN_TOK;
   if (w.N % COLS != 0 || w.K % 128 != 0 || w.E != 1) return I4_ERR_SHAPE;
+  if (linear_big(XT, M, w.N)) return launch_tile_gemm_linear<XT, ST>(x, M, w, bias, y, ot, s);
   const int ks = linear_ksplit(M, w.N, w.K);
   if (ks > 1 && (!ws || ws_bytes < linear_tile_workspace_bytes(M, w.N, w.K)))
     return I4_ERR_WORKSPACE;
@@ -860,12 +718,7 @@ int launch_mfma_linear(const void* x, int M, const TW& w, const void* bias, void
   else I4_LIN(false);
 #undef I4_LIN
   if (hipGetLastError() != hipSuccess) return I4_ERR_LAUNCH;
-  if (ks > 1) {
-    const int64_t total = (int64_t)M * w.N;
-    hipLaunchKernelGGL(k_linear_finish, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                       (const float*)ws, ks, total, w.N, bias, y, ot);
-    if (hipGetLastError() != hipSuccess) return I4_ERR_LAUNCH;
-  }
+  if (ks > 1) return launch_linear_finish((const float*)ws, ks, M, w.N, bias, y, ot, s);
   return I4_OK;
 }
 

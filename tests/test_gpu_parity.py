@@ -438,6 +438,60 @@ def test_linear_tile_rows(pkg, dev, M, N, fmt):
     assert i4ref.rel_err(got, rows) <= TOL
 
 
+def _ct_or_awq(pkg, dev, rng, E, N, K, fmt):
+    """(QWeight, dequantised float64 rows of expert e, activation dtype) of a named format."""
+    kind, g, xdt = fmt.split("-")
+    G = int(g[1:])
+    if kind == "awq":
+        qw, qz, sc = _gen.awq_weight(rng, E, K, N, G, np.float16 if xdt == "f16" else "bf16")
+        return (pkg.QWeight(t_(qw, dev), t_(sc, dev), t_(qz, dev), "awq", G, N, K).to_ct(),
+                lambda e: i4ref.awq_dequant(qw[e], qz[e], f_(sc[e]), G), xdt)
+    p, sc, _ = _gen.ct_weight(rng, E, N, K, G, sdt=np.float16 if xdt == "f16" else "bf16")
+    return (pkg.QWeight(t_(p, dev), t_(sc, dev), None, "ct", G, N, K),
+            lambda e: i4ref.ct_dequant(p[e], f_(sc[e]), K, G), xdt)
+
+
+BIG_FMTS = ["ct-g32-bf16", "awq-g32-bf16", "awq-g128-bf16", "awq-g128-f16", "ct-g64-f16"]
+
+
+@pytest.mark.parametrize("fmt", BIG_FMTS)
+@pytest.mark.parametrize("M,K", [(2048, 128), (1921, 384)])
+def test_linear_128_row_tiles(pkg, dev, fmt, M, K):
+    """Enough rows for the 128 x 256 tiles (2048 -> 4096 outputs: 256 of them), a ragged last
+    tile of one row and an odd number of superchunks, against the oracle's float64 matmul."""
+    rng = np.random.default_rng(M + K)
+    w, dq, xdt = _ct_or_awq(pkg, dev, rng, 1, 4096, K, fmt)
+    x = make_x(rng, (M, K), xdt)
+    got = host(pkg.ops.linear(t_(x, dev), w.to_tile()))
+    assert i4ref.rel_err(got, f_(x) @ dq(0).T) <= MOE_TOL[xdt]
+
+
+@pytest.mark.parametrize("fmt", BIG_FMTS)
+@pytest.mark.parametrize("T", [1025, 4100])
+def test_moe_128_token_tiles(pkg, dev, fmt, T):
+    """Calls of more than 1024 tokens run on 128-token tiles in passes of 4096: experts with 0,
+    1, 16, 17, 33, 65, 128, 129 and 257 tokens in a pass, and a last pass of four tokens."""
+    rng = np.random.default_rng(47 + T)
+    E, H, I, k = 24, 256, 128, 8
+    gu, dgu, xdt = _ct_or_awq(pkg, dev, rng, E, 2 * I, H, fmt)
+    dn, ddn, _ = _ct_or_awq(pkg, dev, rng, E, H, I, fmt)
+    sizes = {0: 0, 1: 1, 2: 16, 3: 17, 4: 33, 5: 65, 6: 128, 7: 129, 8: 257}
+    lg = rng.uniform(-4.0, -1.0, (T, E))
+    lg[:, 0] = -8.0
+    fill = 9
+    for t in range(T):
+        chosen = [e for e, n in sizes.items() if t < n][:k]
+        while len(chosen) < k:
+            chosen.append(fill)
+            fill = 9 + (fill - 9 + 1) % (E - 9)
+        lg[t, chosen] = 2.0 + 0.0625 * rng.permutation(k)
+    lg = i4ref.f32_to_bf16_bits(lg.astype(np.float32)) if xdt == "bf16" else lg.astype(np.float16)
+    wr = np.zeros((E, H), np.float16)
+    moe = pkg.FusedPackedMoE.from_stacked(gu, dn, t_(wr, dev), top_k=k)
+    x = make_x(rng, (T, H), xdt)
+    _check_moe(pkg, moe, dgu, ddn, x, xdt, dev, logits=lg, residual=x)
+
+
 def test_packed_qkv_matches_three_linears(pkg, dev):
     """q, k, v in one launch equal the three separate launches bit for bit (each row's dot
     product does not depend on its neighbours): AWQ parts, and CT parts with and without
