@@ -186,9 +186,11 @@ int    i4_dq_gemv_bounded(const void* x, int x_dtype, int64_t x_stride,
  * tile kernel over 64-row tiles, each weight tile streamed once per 64 rows
  * (the path for prefill and other M > 1 batches); when that grid is small it
  * is split along K into fp32 partials in the workspace and summed in a fixed
- * order.  i4_linear_workspace_bytes gives the workspace (0: none needed); for
- * an AWQ weight it is i4_dq_gemv's split-K workspace (M <= 8), with its status
- * word. */
+ * order.  i4_linear_workspace_bytes gives the workspace (0: none needed).  An
+ * AWQ weight runs the GEMV for a few rows (i4_dq_gemv's split-K workspace, with
+ * its status word) and MFMA straight on the AWQ words from 4 rows (6 below 1024
+ * outputs) on, split along K into partials kept behind the GEMV's part of the
+ * workspace; without that workspace the GEMV runs for every row. */
 int    i4_linear(const void* x, int x_dtype, int M, const i4_qweight* w,
                  const void* bias, void* y, int y_dtype,
                  void* workspace, size_t workspace_bytes, hipStream_t stream);

@@ -797,6 +797,19 @@ static AwqSplit awq_split_plan(const i4_qweight& w, int k_sel) {
   return p;
 }
 
+// Rows of x from which an in-place AWQ linear runs on MFMA (i4_awq_mm.hip) instead of the
+// GEMV, which streams the weight once per row.  us, GEMV / MFMA, back to back in a graph:
+// 2048 -> 4096 2 rows 6.2 / 6.3, 4 rows 8.7 / 6.6; 4096 -> 2048 4 rows 10.7 / 7.3; 2048 ->
+// 768 4 rows 5.9 / 6.4, 8 rows 8.7 / 6.6; 2048 -> 512 4 rows 5.1 / 6.4, 8 rows 8.5 / 6.5.
+static int awq_mm_rows(int N) { return N >= 1024 ? 4 : 6; }
+// Its fp32 partials stay clear of the split-K GEMV's (value, tag) pairs, whose tags must
+// not be met by chance, so that one workspace serves calls of any number of rows.
+static constexpr size_t MM_OFFSET = SK_HEAD + kSplitBytes;
+static size_t awq_mm_bytes(const i4_qweight& w, int M) {
+  const int ks = awq_mm_fits(M, w.N, w.K) ? awq_mm_ksplit(M, w.N, w.K) : 1;
+  return ks > 1 ? MM_OFFSET + (size_t)ks * M * w.N * sizeof(float) : 0;
+}
+
 // the tag of one call of the split-K GEMV: a process-wide count, never 0
 static std::atomic<uint32_t> g_call_tag{0};
 static u32 next_call_tag() {
@@ -922,6 +935,10 @@ int i4_rmsnorm_linear(const void* x, int x_dtype, int M, const void* norm_w, flo
 
 size_t i4_linear_workspace_bytes(const i4_qweight* w, int M) {
   if (w && w->layout == I4_LAYOUT_TILE && M >= 1) return linear_tile_workspace_bytes(M, w->N, w->K);
+  i4_qweight nw;
+  if (w && i4_check_weight(w, &nw) == I4_OK && nw.layout == I4_LAYOUT_AWQ &&
+      M >= awq_mm_rows(nw.N))
+    return awq_mm_bytes(nw, M);
   return i4_dq_gemv_workspace_bytes(w, M);
 }
 
@@ -951,6 +968,19 @@ int i4_linear(const void* x, int x_dtype, int M, const i4_qweight* w, const void
   if (nw.layout == I4_LAYOUT_CT)
     return i4_launch_gemv_ct(x, x_dtype, nw.K, &nw, nullptr, M, y, y_dtype, bias, stream);
   if (!awq_scales_aligned(nw)) return I4_ERR_ALIGN;
+  if (M >= awq_mm_rows(nw.N) && awq_mm_fits(M, nw.N, nw.K)) {
+    const size_t need = awq_mm_bytes(nw, M);
+    // without the workspace the GEMV runs, as for every number of rows
+    if (!need || (workspace && workspace_bytes >= need && !((uintptr_t)workspace & 255))) {
+      float* part = need ? (float*)((char*)workspace + MM_OFFSET) : nullptr;
+#define I4_MM_DT(XT_, ST_)                               \
+  if (x_dtype == XT_ && nw.scale_dtype == ST_)           \
+    return launch_awq_mm<XT_, ST_>(x, M, nw, bias, y, y_dtype, part, stream);
+      I4_MM_DT(I4_F16, I4_F32) I4_MM_DT(I4_F16, I4_F16) I4_MM_DT(I4_F16, I4_BF16)
+      I4_MM_DT(I4_BF16, I4_F32) I4_MM_DT(I4_BF16, I4_F16) I4_MM_DT(I4_BF16, I4_BF16)
+#undef I4_MM_DT
+    }
+  }
   return launch_gemv_awq(x, x_dtype, nw.K, &nw, nullptr, M, y, y_dtype, bias, workspace,
                          workspace_bytes, stream);
 }

@@ -438,6 +438,37 @@ def test_linear_tile_rows(pkg, dev, M, N, fmt):
     assert i4ref.rel_err(got, rows) <= TOL
 
 
+@pytest.mark.parametrize("xdt,sdt,G", [("f16", np.float16, 128), ("bf16", "bf16", 32),
+                                       ("f16", np.float32, 64)])
+@pytest.mark.parametrize("M,N,K", [(9, 2048, 4096), (16, 72, 96), (17, 264, 256), (33, 128, 1024),
+                                   (70, 768, 2048)])
+def test_linear_awq_rows(pkg, dev, M, N, K, xdt, sdt, G):
+    """Several rows on AutoAWQ weights in place run on MFMA: ragged row blocks, columns that
+    end inside a 128-column strip, fewer steps of 32 than waves, K split or not; with the
+    module's workspace, and without any (the GEMV), against the float64 matmul."""
+    rng = np.random.default_rng(M + N + K)
+    qw, qz, sc = _gen.awq_weight(rng, 1, K, N, G, sdt)
+    W = i4ref.awq_dequant(qw, qz, f_(sc), G)[0]
+    w = pkg.QWeight(t_(qw, dev), t_(sc, dev), t_(qz, dev), "awq", G, N, K)
+    x = make_x(rng, (M, K), xdt)
+    bias = make_x(rng, (N,), xdt)
+    ref = f_(x) @ W.T + f_(bias)
+    lin = pkg.PackedLinear.from_qweight(w, t_(bias, dev), repack=False)
+    got = lin(t_(x, dev))
+    # one rounding of the output (2^-9 bf16, 2^-12 fp16 of the value) over fp32 sums
+    assert i4ref.rel_err(host(got), ref) <= MOE_TOL[xdt]
+    assert torch.equal(lin(t_(x, dev)), got)
+    one = host(lin(t_(x[:1], dev)))  # the same workspace serves the GEMV in between
+    assert i4ref.rel_err(one, ref[:1]) <= MOE_TOL[xdt]
+    y = torch.empty_like(got)
+    cw, xd, bd = w.c(), t_(x, dev), t_(bias, dev)
+    lb = pkg.lib()
+    code = {"f16": 1, "bf16": 2}[xdt]
+    assert lb.i4_linear(xd.data_ptr(), code, M, ctypes.byref(cw), bd.data_ptr(), y.data_ptr(),
+                        code, None, 0, torch.cuda.current_stream().cuda_stream) == 0
+    assert i4ref.rel_err(host(y), ref) <= MOE_TOL[xdt]
+
+
 def _ct_or_awq(pkg, dev, rng, E, N, K, fmt):
     """(QWeight, dequantised float64 rows of expert e, activation dtype) of a named format."""
     kind, g, xdt = fmt.split("-")
