@@ -8,6 +8,7 @@
 // ranking the probabilities.  Exact ties are broken by the lower expert id
 // (torch.topk leaves that order unspecified).
 #include "i4_common.h"
+#include "i4_halve.h"
 #include "i4_router_body.h"
 #include "i4_launch.h"
 #include "i4_topk.h"
@@ -335,6 +336,68 @@ __global__ __launch_bounds__(256) void k_router_t(const uint16_t* __restrict__ x
   });
 }
 
+// The logits of many tokens, H = 512 NR <= 2048.  A wave holds eight router rows in
+// registers (32 experts per workgroup) while `stages` times eight tokens pass by in LDS;
+// the next eight are loaded during the products.  A logit is k_router_t's lane chain, and
+// the halving butterfly adds the lanes as its wave sum does: the same bits.  Bound: the
+// dot2 rate.  k_router_t spends as much on its 64 six-step wave sums per 8 x 8 tile, one
+// finished value each, as on the products; us, there / here: 512 tokens of H 2048 17.6 /
+// 7.4, 3001 tokens 69 / 25, 700 tokens of H 1024 15.8 / 6.2.
+template <int XT, int NR>
+__global__ __launch_bounds__(256) void k_router_g(const uint16_t* __restrict__ x, int T,
+                                                  const uint16_t* __restrict__ wr, int E,
+                                                  int stages, uint16_t* __restrict__ logits) {
+  constexpr int H = 512 * NR, WORDS = 64 * NR, NS = 8 * WORDS / 256;
+  __shared__ u32x4 s_x[8 * WORDS];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int e0 = ((int)blockIdx.x * 4 + wave) * 8, t_lo = (int)blockIdx.y * stages * 8;
+  const int t_hi = min(T, t_lo + stages * 8);
+  u32x4 sv[NS];
+  auto load = [&](int t0) {
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      const int i = tid + 256 * u, tk = i / WORDS;
+      sv[u] = ldg16(x + (int64_t)min(t0 + tk, T - 1) * H + 8 * (i - tk * WORDS));
+    }
+  };
+  load(t_lo);
+  u32x4 wv[8][NR];
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      wv[r][i] = ldg16(wr + (int64_t)min(e0 + r, E - 1) * H + 8 * lane + 512 * i);
+  for (int t0 = t_lo; t0 < t_hi; t0 += 8) {
+    __syncthreads();  // the previous tokens are read
+#pragma unroll
+    for (int u = 0; u < NS; ++u) s_x[tid + 256 * u] = sv[u];
+    __syncthreads();
+    if (t0 + 8 < t_hi) load(t0 + 8);
+    float pv[8];
+#pragma unroll
+    for (int tk = 0; tk < 8; ++tk) {
+      float a[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) a[r] = 0.f;
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const u32x4 xw = s_x[tk * WORDS + lane + 64 * i];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          a[r] = Half<XT>::dot2(wv[r][i].x, xw.x, a[r]);
+          a[r] = Half<XT>::dot2(wv[r][i].y, xw.y, a[r]);
+          a[r] = Half<XT>::dot2(wv[r][i].z, xw.z, a[r]);
+          a[r] = Half<XT>::dot2(wv[r][i].w, xw.w, a[r]);
+        }
+      }
+      pv[tk] = halve_rows(a, lane);
+    }
+    const float v = halve_tokens(pv, lane);
+    const int t = t0 + (lane >> 3), e = e0 + (lane & 7);
+    if (t < t_hi && e < E) logits[(int64_t)t * E + e] = Half<XT>::from_f32(v);
+  }
+}
+
 // Tag of the routing words of one call at workspace epoch e: odd, so a zero-filled
 // buffer never matches.
 __device__ inline u32 route_tag(u32 e) { return (2u * e + 1u) * 0x9E3779B1u; }
@@ -474,6 +537,20 @@ int i4_launch_router_logits(const void* x, int xt, int T, int H, const void* wr,
   }
     if (T <= 64) {
       I4_RT_CASE(I4_F16, 1, 1) else I4_RT_CASE(I4_BF16, 1, 1)
+    } else if (H % 512 == 0 && H <= 2048) {
+      // eight tokens per workgroup until the chip is filled twice, then more (each
+      // workgroup reads its 32 router rows once)
+      const int eg = (E + 31) / 32;
+      int stages = (int)((int64_t)T * eg / (8 * 512));
+      stages = stages < 1 ? 1 : stages > 8 ? 8 : stages;
+      const dim3 g3(eg, (T + 8 * stages - 1) / (8 * stages));
+#define I4_RG_CASE(XT_, NR_)                                                                  \
+  if (xt == XT_ && H == 512 * NR_)                                                            \
+    hipLaunchKernelGGL((k_router_g<XT_, NR_>), g3, dim3(256), 0, s, xin, T,                   \
+                       (const uint16_t*)wr, E, stages, (uint16_t*)logits);
+      I4_RG_CASE(I4_F16, 1) I4_RG_CASE(I4_F16, 2) I4_RG_CASE(I4_F16, 3) I4_RG_CASE(I4_F16, 4)
+      I4_RG_CASE(I4_BF16, 1) I4_RG_CASE(I4_BF16, 2) I4_RG_CASE(I4_BF16, 3) I4_RG_CASE(I4_BF16, 4)
+#undef I4_RG_CASE
     } else {
       I4_RT_CASE(I4_F16, 8, 2) else I4_RT_CASE(I4_BF16, 8, 2)
     }

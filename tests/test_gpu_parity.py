@@ -1214,6 +1214,20 @@ def test_router_tokens_match_single_token_bits(pkg, dev, xdt, norm, H):
             assert torch.equal(one[0], full[t])
 
 
+@pytest.mark.parametrize("xdt", ["f16", "bf16"])
+@pytest.mark.parametrize("T,E,H", [(65, 128, 2048), (131, 40, 1024), (67, 5, 512), (70, 128, 1536),
+                                   (2101, 128, 1024)])
+def test_router_many_tokens_match_few_bits(pkg, dev, xdt, T, E, H):
+    """More than 64 tokens (eight expert rows per wave, tokens in passes of eight, several
+    passes per workgroup at 2101; ragged tokens and experts): the logits of calls of at most
+    64 tokens, bit for bit."""
+    rng = np.random.default_rng(T + H)
+    wr = t_(make_x(rng, (E, H), xdt), dev) * 0.05
+    x = t_(make_x(rng, (T, H), xdt), dev)
+    few = torch.cat([pkg.router_logits(x[i:i + 64], wr) for i in range(0, T, 64)])
+    assert torch.equal(pkg.router_logits(x, wr), few)
+
+
 def test_graph_replays_match_eager(pkg, dev):
     rng = np.random.default_rng(28)
     moe, _, _, _ = _awq_moe(pkg, dev, rng, E=32)
