@@ -19,7 +19,8 @@
 // instead of once per token (the reference loops over tokens,
 // fused_packed_moe.py:231).  With T <= 64 every expert is cut into small
 // entries and the large-entry launches are skipped.  The MFMA kernels are in
-// i4_moe_mfma.hip.
+// i4_moe_mfma.hip.  More than 1024 tokens run in passes of up to 4096 on the 128-token
+// tiles of i4_tile_gemm.hip, grouped by k_group_e (tile_gemm_fits).
 #include "i4_common.h"
 #include "i4_launch.h"
 #include "i4_moe_launch.h"
@@ -35,32 +36,45 @@ static constexpr int BIG_CHUNK = 4096;  // and by one of the passes on 128-token
 // in the activation dtype (each expert's output rounded as the reference rounds
 // it, fused_packed_moe.py:262; half the bytes of fp32 through HBM), the sum in
 // fp32.  KMAX >= topk slots are loaded unconditionally (indices clamped) so that
-// all loads of a thread are in flight together.
-template <int XT, int KMAX>
+// all loads of a thread are in flight together.  V values per thread (H % V == 0, rows
+// 2 V-byte aligned).  Bound: HBM; one value per thread left it at 3.3 TB/s (3001 tokens
+// 30 us, 20 with four).
+template <int XT, int KMAX, int V>
 __global__ __launch_bounds__(WG) void k_moe_combine(const uint16_t* __restrict__ ys,
                                                     const float* __restrict__ wts,
                                                     const int32_t* __restrict__ sel, int T,
                                                     int topk, int E, int H,
                                                     const uint16_t* __restrict__ residual,
                                                     uint16_t* __restrict__ out) {
-  const int64_t i = min((int64_t)blockIdx.x * WG + threadIdx.x, (int64_t)T * H - 1);
+  struct alignas(2 * V) Vec { uint16_t h[V]; };
+  const int64_t q = (int64_t)blockIdx.x * WG + threadIdx.x;
+  if (q * V >= (int64_t)T * H) return;
+  const int64_t i = q * V;
   const int t = (int)(i / H), n = (int)(i - (int64_t)t * H);
-  const uint16_t rraw = *(residual ? residual + i : (const uint16_t*)sel);
+  const Vec rr = *(const Vec*)((residual ? residual : ys) + i);  // no branch before the loads
+  Vec yv[KMAX];
   int sl[KMAX];
-  float wv[KMAX], yv[KMAX];
+  float wv[KMAX];
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
     const int s = t * topk + min(j, topk - 1);
     sl[j] = sel[s];
     wv[j] = wts[s];
-    yv[j] = Half<XT>::to_f32(ys[(int64_t)s * H + n]);
+    yv[j] = *(const Vec*)(ys + (int64_t)s * H + n);
   }
-  float y = 0.f;
+  Vec o;
 #pragma unroll
-  for (int j = 0; j < KMAX; ++j)
-    if (j < topk) y += wv[j] * ((unsigned)sl[j] < (unsigned)E ? yv[j] : __builtin_nanf(""));
-  const float r = residual ? Half<XT>::to_f32(rraw) : 0.f;
-  if ((int64_t)blockIdx.x * WG + threadIdx.x < (int64_t)T * H) out[i] = Half<XT>::from_f32(r + y);
+  for (int v = 0; v < V; ++v) {
+    float y = 0.f;
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j)
+      if (j < topk)
+        y += wv[j] * ((unsigned)sl[j] < (unsigned)E ? Half<XT>::to_f32(yv[j].h[v])
+                                                     : __builtin_nanf(""));
+    const float r = residual ? Half<XT>::to_f32(rr.h[v]) : 0.f;
+    o.h[v] = Half<XT>::from_f32(r + y);
+  }
+  *(Vec*)(out + i) = o;
 }
 
 
@@ -569,18 +583,18 @@ int moe_chunk(const void* x, int xt, int T, const i4_moe_weights* mw, const i4_q
                         ws.entries, ws.n_entries, ws.perm, tdn, I, ws.ys, s);
     if (rc) return rc;
   }
-  const int64_t tot = (int64_t)T * H;
+  // four values per thread; up to 64 tokens, where the launch does not fill the chip, one
+  const int V = T <= ONE_LIST_T ? 1 : 4;
+  const int64_t tot = (int64_t)T * H / V;
   dim3 cg((unsigned)((tot + WG - 1) / WG));
-#define I4_COMB_CASE(XT_, KM_)                                                                 \
-  hipLaunchKernelGGL((k_moe_combine<XT_, KM_>), cg, dim3(WG), 0, s, (const uint16_t*)ws.ys, wts, \
-                     sel, T, topk, E, H, (const uint16_t*)residual, (uint16_t*)out)
-  if (xt == I4_F16) {
-    if (topk <= 8) I4_COMB_CASE(I4_F16, 8);
-    else I4_COMB_CASE(I4_F16, 16);
-  } else {
-    if (topk <= 8) I4_COMB_CASE(I4_BF16, 8);
-    else I4_COMB_CASE(I4_BF16, 16);
-  }
+#define I4_COMB_CASE(XT_, KM_, V_)                                                             \
+  if (xt == XT_ && (topk <= 8) == (KM_ == 8) && V == V_)                                       \
+  hipLaunchKernelGGL((k_moe_combine<XT_, KM_, V_>), cg, dim3(WG), 0, s, (const uint16_t*)ws.ys, \
+                     wts, sel, T, topk, E, H, (const uint16_t*)residual, (uint16_t*)out);
+  I4_COMB_CASE(I4_F16, 8, 1) I4_COMB_CASE(I4_F16, 8, 4)
+  I4_COMB_CASE(I4_F16, 16, 1) I4_COMB_CASE(I4_F16, 16, 4)
+  I4_COMB_CASE(I4_BF16, 8, 1) I4_COMB_CASE(I4_BF16, 8, 4)
+  I4_COMB_CASE(I4_BF16, 16, 1) I4_COMB_CASE(I4_BF16, 16, 4)
 #undef I4_COMB_CASE
   return hipGetLastError() == hipSuccess ? I4_OK : I4_ERR_LAUNCH;
 }
