@@ -7,8 +7,12 @@
 // merged byte-wise with v_perm_b32, as in the AWQ GEMVs).  Step s then is eight MFMAs, one
 // per nibble slot, each over 16 columns eight apart: a wave covers 128 columns x 16 MB rows
 // x 32 k.  A operands come straight from x.
-//   fp16: B = q - z exactly.  bf16: B = M + q exactly and an MFMA with ones gives S_m, the
-//   sum of row m's activations, in the accumulator's own layout: s (D - (M + z) S_m).
+//   fp16: B = q - z exactly.  bf16: B = 16 + q exactly (a nibble in the mantissa's upper
+//   bits) and an MFMA with ones gives S_m, the sum of row m's activations, in the
+//   accumulator's own layout: s (D - (16 + z) S_m).  The difference cancels and leaves the
+//   rounding of the two terms, which grows with the bias: 24 rows, 4096 -> 2048, groups of
+//   128, relative 2-norm of the fp32 result against float64: 5.5e-7 with 128 + q (one
+//   operation per nibble pair less), 1.0e-7 with 16 + q; the GEMV 2.2e-7.
 // Every group's sums are scaled in fp32, as in the GEMVs: the same precision.
 //
 // The GEMVs above stream the weight once per row of x (24 rows of 4096 -> 2048: 97 us, 105
@@ -48,7 +52,7 @@ __global__ __launch_bounds__(256) void k_awq_mm(
   // steps of this workgroup, then of this wave
   const int S = K >> 5, a0 = kz * S / ksplit, na = (kz + 1) * S / ksplit - a0;
   const int s_lo = a0 + na * wave / 4, s_hi = a0 + na * (wave + 1) / 4;
-  const u32 mg = magic_v<XT>();
+  const u32 mg = F16 ? magic_v<XT>() : vgpr_const(0x41804180u);  // bf16: 16 twice
   constexpr u32 ONE2 = 0x3F803F80u;
   const u32x4 ones = {ONE2, ONE2, ONE2, ONE2};
   // the expert's weight and a row block of x are below 2^31 bytes (checked on the host)
@@ -97,10 +101,13 @@ __global__ __launch_bounds__(256) void k_awq_mm(
       for (int q = 0; q < 4; ++q) {
         const u32 sel = 0x0C000C00u | (u32)q | ((u32)(4 + q) << 16);
         const u32 t = __builtin_amdgcn_perm(o.w[2 * p + 1], o.w[2 * p], sel);
-        u32 lo = (t & 0x000F000Fu) | mg, hi = ((t >> 4) & 0x000F000Fu) | mg;
+        u32 lo, hi;
         if constexpr (F16) {
-          lo = sub_zero(lo, nz[2 * q]);
-          hi = sub_zero(hi, nz[2 * q + 1]);
+          lo = sub_zero((t & 0x000F000Fu) | mg, nz[2 * q]);
+          hi = sub_zero(((t >> 4) & 0x000F000Fu) | mg, nz[2 * q + 1]);
+        } else {
+          lo = ((t << 3) & 0x00780078u) | mg;
+          hi = ((t >> 1) & 0x00780078u) | mg;
         }
         bo[2 * q][p] = lo;
         bo[2 * q + 1][p] = hi;
@@ -117,7 +124,7 @@ __global__ __launch_bounds__(256) void k_awq_mm(
 #pragma unroll
     for (int sl = 0; sl < 8; ++sl) {
       const float sv = scale_from_raw<ST>(sr[sl]);
-      const float mz = Half<XT>::MAGIC + (float)((zw >> (4 * sl)) & 15u);
+      const float mz = 16.f + (float)((zw >> (4 * sl)) & 15u);  // bf16
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
