@@ -15,6 +15,7 @@ import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "libi4moe.so"
 ABI_VERSION = 9
+ERR_HANDOFF = -10  # I4_ERR_HANDOFF: the one code a kernel stores in a status word
 
 # element types and layouts (include/i4moe.h)
 F32, F16, BF16 = 0, 1, 2

@@ -52,8 +52,7 @@ def gemv_status(workspace: "Workspace | None" = None, device: torch.device | Non
         workspace = _STREAM_WS.get((dev.index, _lib.stream(dev), "awq"))
     if workspace is None or workspace.buf is None:
         return 0
-    torch.cuda.synchronize(workspace.buf.device)
-    return int(workspace.buf[:4].view(torch.int32).item())
+    return _status_word(workspace, 0)
 
 
 def dequant_gemv(x, packed, scale, sel, group=32, block_r=64, nw_blk=8, *, zeros=None,
@@ -269,18 +268,49 @@ def moe_weights_c(gate_up: QWeight, down: QWeight, router_w: torch.Tensor | None
     return mw
 
 
+def _capturing(device: torch.device) -> bool:
+    return device.type == "cuda" and torch.cuda.is_current_stream_capturing()
+
+
 class Workspace:
-    """Grow-only device scratch for the MoE entry points (one per module)."""
+    """Grow-only device scratch for the MoE entry points (one per module).
+
+    A buffer handed out under stream capture belongs to that graph: every replay writes to
+    it.  When a later call needs more, such a buffer is kept as long as this object lives
+    instead of going back to the allocator, and its successor is at least twice as large,
+    so the kept ones never add up to more than the one in use."""
 
     def __init__(self) -> None:
         self.buf: torch.Tensor | None = None
+        self.kept: list[torch.Tensor] = []
+        self._captured = False  # whether self.buf was handed out under capture
 
     def get(self, nbytes: int, device: torch.device, zeroed: bool = False) -> torch.Tensor:
         """At least nbytes; zeroed: a new buffer is allocated as zeros."""
         if self.buf is None or self.buf.numel() < nbytes or self.buf.device != device:
+            if self._captured:
+                self.kept.append(self.buf)
+                nbytes = max(nbytes, 2 * self.buf.numel())
+                self._captured = False
             make = torch.zeros if zeroed else torch.empty
             self.buf = make(max(nbytes, 1), dtype=torch.uint8, device=device)
+        if not self._captured:
+            self._captured = _capturing(device)
         return self.buf
+
+
+def _status_word(workspace: Workspace, off: int) -> int:
+    """The int32 at byte off of the workspace's buffer, or the I4_ERR_HANDOFF code when a
+    graph's replay left it in a buffer kept for that graph; synchronises the device."""
+    if workspace.buf is None or workspace.buf.numel() < off + 4:
+        raise RuntimeError("the workspace has not served a call of these sizes")
+    torch.cuda.synchronize(workspace.buf.device)
+    word = int(workspace.buf[off:off + 4].view(torch.int32).item())
+    for buf in getattr(workspace, "kept", ()):
+        if word == 0 and buf.numel() >= off + 4:
+            old = int(buf[off:off + 4].view(torch.int32).item())
+            word = old if old == _lib.ERR_HANDOFF else 0
+    return word
 
 
 def moe_forward(x: torch.Tensor, gate_up: QWeight, down: QWeight, top_k: int,
@@ -348,10 +378,7 @@ def moe_status(workspace: Workspace, T: int, H: int, I: int, E: int, top_k: int)
     """The status word the last i4_moe_forward / stack call with this workspace left
     (0, or the I4_ERR_HANDOFF code when a decode wait gave up); synchronises the device."""
     off = _lib.lib().i4_moe_status_offset(T, H, I, E, top_k)
-    if workspace.buf is None or workspace.buf.numel() < off + 4:
-        raise RuntimeError("the workspace has not served a call of these sizes")
-    torch.cuda.synchronize(workspace.buf.device)
-    return int(workspace.buf[off:off + 4].view(torch.int32).item())
+    return _status_word(workspace, off)
 
 
 def moe_down_wait(act: torch.Tensor, down: QWeight, logits: torch.Tensor, top_k: int,
@@ -689,10 +716,7 @@ def attn_status(workspace: Workspace, n_heads: int, head_dim: int, max_len: int)
     """The status word the last attn_decode_o call with this workspace left (0, or the
     I4_ERR_HANDOFF code when an o_proj wait gave up); synchronises the device."""
     off = _lib.lib().i4_attn_decode_o_status_offset(n_heads, head_dim, max_len)
-    if workspace.buf is None or workspace.buf.numel() < off + 4:
-        raise RuntimeError("the workspace has not served a call of these sizes")
-    torch.cuda.synchronize(workspace.buf.device)
-    return int(workspace.buf[off:off + 4].view(torch.int32).item())
+    return _status_word(workspace, off)
 
 
 def thinker_layer_fits(n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, H: int,
@@ -879,10 +903,7 @@ def dmoe_status(workspace: Workspace, T: int, E: int, top_k: int, I: int, Is: in
     I4_ERR_HANDOFF code when a down workgroup of the single-launch decode block gave up
     waiting for its activations); synchronises the device."""
     off = _lib.lib().i4_dmoe_status_offset(T, E, top_k, I, Is)
-    if workspace.buf is None or workspace.buf.numel() < off + 4:
-        raise RuntimeError("the workspace has not served a call of these sizes")
-    torch.cuda.synchronize(workspace.buf.device)
-    return int(workspace.buf[off:off + 4].view(torch.int32).item())
+    return _status_word(workspace, off)
 
 
 def dmoe_down_wait(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top_k: int,
