@@ -120,9 +120,10 @@ def dequant_gemv_bounded(x: torch.Tensor, w: QWeight, sel: torch.Tensor, max_pol
 def linear(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
            out_dtype: torch.dtype | None = None,
            workspace: "Workspace | None" = None) -> torch.Tensor:
-    """y = x W^T (+ bias) for every row of x in one launch (E = 1 weight).  workspace: kept
-    by the caller for the calls that need one (an AWQ weight split along K, a tile weight
-    split along K); by default one per device and stream."""
+    """y = x W^T (+ bias) for every row of x (E = 1 weight), in one launch or, where K is split
+    into partial sums, two.  workspace: kept by the caller for the calls that need one (a few
+    rows on an AWQ weight split along K, a tile weight split along K); by default one per
+    device and stream.  Several rows on an AWQ weight allocate their partials per call."""
     dev = _lib.require_device(x, w.packed, bias)
     xt = _lib.half_code(x.dtype)
     lead = x.shape[:-1]
@@ -139,7 +140,16 @@ def linear(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
             raise RuntimeError("bias length != out_features")
     lb = _lib.lib()
     cw = w.c()
-    ws = _gemv_ws(lb.i4_linear_workspace_bytes(ctypes.byref(cw), M), dev, workspace, w.layout)
+    nbytes = lb.i4_linear_workspace_bytes(ctypes.byref(cw), M)
+    # (the GEMV splits K for at most 8 rows)
+    if w.layout == "awq" and nbytes and (
+            M > 8 or nbytes != lb.i4_dq_gemv_workspace_bytes(ctypes.byref(cw), M)):
+        # several rows on MFMA: the partial sums live from one launch of the call to the next
+        # only, so they take memory of the call's stream (or graph) and not the kept
+        # workspace, which other streams and captured calls of fewer rows may be using
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    else:
+        ws = _gemv_ws(nbytes, dev, workspace, w.layout)
     _lib.check(lb.i4_linear(flat.data_ptr(), xt, M, ctypes.byref(cw), _lib.ptr(b), y.data_ptr(),
                             _lib.dtype_code(od), None if ws is None else ws.data_ptr(),
                             0 if ws is None else ws.numel(), _lib.stream(dev)))

@@ -56,3 +56,25 @@ def test_rows_lose_no_precision(pkg, dev, xdt, G, M, N, K):
 
     got = err(pkg.ops.linear(x, w, out_dtype=torch.float32))
     assert got <= 1.2 * err(gemv_rows(pkg, w, x, xdt)), got
+
+
+def test_two_streams_share_one_module(pkg, dev):
+    """Calls of several rows on two streams at once, each with inputs of its own: the results
+    of the same calls one after the other."""
+    rng = np.random.default_rng(71)
+    w, _ = awq(pkg, dev, rng, 2048, 4096, 128, "f16")
+    lin = pkg.PackedLinear.from_qweight(w, repack=False)
+    xs = [[t_(make_x(rng, (rows, 4096), "f16"), dev) for rows in (24, 9, 31, 24)]
+          for _ in range(2)]
+    want = [[lin(x).clone() for x in side] for side in xs]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in xs]
+    got = [[], []]
+    for _ in range(30):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                got[i] += [lin(x) for x in xs[i]]
+    torch.cuda.synchronize()
+    for i in range(2):
+        for n, y in enumerate(got[i]):
+            assert torch.equal(y, want[i][n % 4])

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from tests.test_gpu_awq_rows import awq
 from tests.test_gpu_parity import _awq_moe, make_x, t_
 
 pytestmark = pytest.mark.gpu
@@ -24,7 +25,7 @@ def replay_after_larger(module, small, larger, workspace):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         out = module(static)
-    held = workspace.buf.numel()
+    held = 1 << 23 if workspace.buf is None else workspace.buf.numel()
     for x in larger:
         module(x)
     torch.cuda.synchronize()
@@ -47,3 +48,17 @@ def test_moe_graph_after_larger_calls(pkg, dev, T):
     larger = [t_(make_x(rng, (n, 2048), "f16"), dev) for n in (40, 300)]
     replay_after_larger(moe, small, larger, moe.workspace)
     assert pkg.moe_status(moe.workspace, T, 2048, moe.down.K, 32, moe.top_k) == 0
+
+
+@pytest.mark.parametrize("rows", [1, 4, 12])
+@pytest.mark.parametrize("N,K", [(2048, 4096), (512, 2048)])
+def test_awq_linear_graph_after_larger_calls(pkg, dev, rows, N, K):
+    """One row (the split-K GEMV on the module's workspace) and several rows (partials of the
+    call, here of the graph)."""
+    rng = np.random.default_rng(67 + rows)
+    w, _ = awq(pkg, dev, rng, N, K, 128, "f16")
+    lin = pkg.PackedLinear.from_qweight(w, repack=False)
+    small = [t_(make_x(rng, (rows, K), "f16"), dev) for _ in range(3)]
+    larger = [t_(make_x(rng, (n, K), "f16"), dev) for n in (24, 256)]
+    replay_after_larger(lin, small, larger, lin.workspace)
+    assert pkg.ops.gemv_status(lin.workspace) == 0
