@@ -180,17 +180,20 @@ int    i4_dq_gemv_bounded(const void* x, int x_dtype, int64_t x_stride,
 
 /* TritonPackedLinear.forward (src/duplex/streaming/triton_dequant_gemv.py:151-159):
  *   y[m][n] = sum_k W[n][k] * x[m][k] (+ bias[n]),  m < M, expert 0 of w.
- * One launch for all M rows (the reference launches once per row).  bias is
- * nullable and in y_dtype.  A CT or AWQ weight runs the dequant-GEMV for
- * every row; a weight in I4_LAYOUT_TILE (E = 1, N % 128 == 0) runs the MFMA
- * tile kernel over 64-row tiles, each weight tile streamed once per 64 rows
- * (the path for prefill and other M > 1 batches); when that grid is small it
- * is split along K into fp32 partials in the workspace and summed in a fixed
- * order.  i4_linear_workspace_bytes gives the workspace (0: none needed).  An
- * AWQ weight runs the GEMV for a few rows (i4_dq_gemv's split-K workspace, with
- * its status word) and MFMA straight on the AWQ words from 4 rows (6 below 1024
- * outputs) on, split along K into partials kept behind the GEMV's part of the
- * workspace; without that workspace the GEMV runs for every row. */
+ * All M rows in one launch, or two where K is split into fp32 partials (the
+ * reference launches once per row).  bias is nullable and in y_dtype.  A CT
+ * weight runs the dequant-GEMV for every row.  A weight in I4_LAYOUT_TILE
+ * (E = 1, N % 128 == 0) runs on MFMA tiles of 64 rows, or 128 rows where those
+ * fill the chip, each weight tile streamed once per tile row (the path for
+ * prefill and other M > 1 batches); a small grid is split along K, summed in a
+ * fixed order.  An AWQ weight runs the GEMV for a few rows (i4_dq_gemv's split-K
+ * workspace, with its status word) and MFMA straight on the AWQ words from 4 rows
+ * on, where M N K is large enough to pay for it; its partials lie behind the
+ * GEMV's part of the workspace, and without that workspace the GEMV runs.
+ * i4_linear_workspace_bytes gives the workspace of this M (0: none needed).  It
+ * does not grow with M throughout (few rows are split, many are not), so ask for
+ * each M, or for the largest over those that will be used: a smaller workspace is
+ * no error on AWQ, but the slower GEMV. */
 int    i4_linear(const void* x, int x_dtype, int M, const i4_qweight* w,
                  const void* bias, void* y, int y_dtype,
                  void* workspace, size_t workspace_bytes, hipStream_t stream);

@@ -797,16 +797,32 @@ static AwqSplit awq_split_plan(const i4_qweight& w, int k_sel) {
   return p;
 }
 
-// Rows of x from which an in-place AWQ linear runs on MFMA (i4_awq_mm.hip) instead of the
-// GEMV, which streams the weight once per row.  us, GEMV / MFMA, back to back in a graph:
-// 2048 -> 4096 2 rows 6.2 / 6.3, 4 rows 8.7 / 6.6; 4096 -> 2048 4 rows 10.7 / 7.3; 2048 ->
-// 768 4 rows 5.9 / 6.4, 8 rows 8.7 / 6.6; 2048 -> 512 4 rows 5.1 / 6.4, 8 rows 8.5 / 6.5.
-static int awq_mm_rows(int N) { return N >= 1024 ? 4 : 6; }
+// Whether an in-place AWQ linear of M rows runs on MFMA (i4_awq_mm.hip) instead of the GEMV,
+// which streams the weight once per row.  MFMA with its summing launch takes 6 us however
+// little there is to do; the line is where the GEMV takes as long, measured over 10 K of
+// 256 .. 8192, 12 N of 64 .. 8192, 4 .. 150 rows, fp16 and bf16, groups of 32, 64 and 128
+// (back to back in a graph): on this side of it no size is over 4 % slower than its GEMV.
+// us, GEMV / MFMA, fp16 in groups of 128:
+//   K-complete GEMV: its time is that of M N K at 2e12 a second over 3.5 us.  2048 -> 128 24
+//   rows 6.1 / 7.9, 768 -> 512 12 rows 5.9 / 6.7, 24 rows 8.2 / 7.7, 4096 -> 2048 24 rows
+//   97 / 10.  Under 256 columns half of the strip pairs idle: 8192 -> 64 32 rows 9.0 / 12.6,
+//   150 rows 27 / 15.
+//   split GEMV (at most 8 rows): narrow slices (short groups) hand more partials over.
+//   2048 -> 2048 4 rows 6.5 / 7.4, 8 rows 9.3 / 7.7, the same in groups of 32 17.7 / 7.3 and
+//   21 / 7.7; 1024 -> 4096 4 rows 6.3 / 6.8, 7 rows 8.2 / 7.1.
+static bool awq_use_mm(const i4_qweight& w, int M) {
+  if (M < 4 || !awq_mm_fits(M, w.N, w.K)) return false;
+  const int64_t work = (int64_t)M * w.N * w.K;
+  const AwqSplit p = awq_split_plan(w, M);
+  if (!p.nwave) return work >= (int64_t)(w.N >= 256 ? 8 : 20) << 20;
+  const int slice = 16 * p.nwave * p.ppt;
+  return M * p.P >= 112 || work >= (int64_t)(slice == 128 ? 24 : slice == 64 ? 12 : 8) << 20;
+}
 // Its fp32 partials stay clear of the split-K GEMV's (value, tag) pairs, whose tags must
 // not be met by chance, so that one workspace serves calls of any number of rows.
 static constexpr size_t MM_OFFSET = SK_HEAD + kSplitBytes;
 static size_t awq_mm_bytes(const i4_qweight& w, int M) {
-  const int ks = awq_mm_fits(M, w.N, w.K) ? awq_mm_ksplit(M, w.N, w.K) : 1;
+  const int ks = awq_mm_ksplit(M, w.N, w.K);
   return ks > 1 ? MM_OFFSET + (size_t)ks * M * w.N * sizeof(float) : 0;
 }
 
@@ -936,9 +952,10 @@ int i4_rmsnorm_linear(const void* x, int x_dtype, int M, const void* norm_w, flo
 size_t i4_linear_workspace_bytes(const i4_qweight* w, int M) {
   if (w && w->layout == I4_LAYOUT_TILE && M >= 1) return linear_tile_workspace_bytes(M, w->N, w->K);
   i4_qweight nw;
-  if (w && i4_check_weight(w, &nw) == I4_OK && nw.layout == I4_LAYOUT_AWQ &&
-      M >= awq_mm_rows(nw.N))
-    return awq_mm_bytes(nw, M);
+  if (w && i4_check_weight(w, &nw) == I4_OK && nw.layout == I4_LAYOUT_AWQ) {
+    nw.E = 1;
+    if (awq_use_mm(nw, M)) return awq_mm_bytes(nw, M);
+  }
   return i4_dq_gemv_workspace_bytes(w, M);
 }
 
@@ -968,7 +985,7 @@ int i4_linear(const void* x, int x_dtype, int M, const i4_qweight* w, const void
   if (nw.layout == I4_LAYOUT_CT)
     return i4_launch_gemv_ct(x, x_dtype, nw.K, &nw, nullptr, M, y, y_dtype, bias, stream);
   if (!awq_scales_aligned(nw)) return I4_ERR_ALIGN;
-  if (M >= awq_mm_rows(nw.N) && awq_mm_fits(M, nw.N, nw.K)) {
+  if (awq_use_mm(nw, M)) {
     const size_t need = awq_mm_bytes(nw, M);
     // without the workspace the GEMV runs, as for every number of rows
     if (!need || (workspace && workspace_bytes >= need && !((uintptr_t)workspace & 255))) {

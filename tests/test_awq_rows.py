@@ -53,3 +53,35 @@ def test_rows_leave_the_kept_workspace_alone(pkg, stub):
         assert ws is None or ws + nbytes <= lo or ws >= hi
     lin(x(1))
     assert stub.calls[-1][1] == lo
+
+
+def _mm_rows(pkg, N, K, G, rows, E=1):
+    """Which of the row counts take partials of the MFMA path (and not the GEMV's workspace)."""
+    import ctypes
+
+    w = awq_linear(pkg, N, K, G).w.c()
+    lb = pkg.lib()
+    size = lambda M: lb.i4_linear_workspace_bytes(ctypes.byref(w), M)
+    return [M for M in rows if size(M) and size(M) != lb.i4_dq_gemv_workspace_bytes(
+        ctypes.byref(w), M)]
+
+
+@pytest.mark.parametrize("N,K,G,first", [
+    # the K-complete GEMV was measured faster below: M N K under 8 M, 20 M below 256 columns
+    (128, 256, 128, None), (128, 2048, 32, 80), (64, 2048, 128, None), (512, 768, 128, 22),
+    (2048, 256, 32, 16), (1024, 256, 64, 32),
+    # against the split GEMV: 112 slices to hand over, or M N K of 24 / 12 / 8 M
+    (2048, 4096, 128, 4), (2048, 2048, 128, 6), (4096, 1024, 128, 6), (512, 2048, 128, 7),
+    (2048, 2048, 64, 4), (2048, 1024, 32, 4), (4096, 768, 64, 4), (64, 8192, 128, 4),
+])
+def test_rows_take_mfma_where_it_was_measured_faster(pkg, N, K, G, first):
+    """The first row count on MFMA; every later one too, up to 8 rows (split GEMV) and from 9
+    (K-complete GEMV) apart."""
+    rows = _mm_rows(pkg, N, K, G, range(1, 160))
+    if first is None:
+        assert not rows
+    else:
+        assert rows[0] == first
+        few, many = [r for r in rows if r <= 8], [r for r in rows if r > 8]
+        for part, last in ((few, 8), (many, 159)):
+            assert not part or part == list(range(part[0], last + 1))

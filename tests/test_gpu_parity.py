@@ -440,8 +440,8 @@ def test_linear_tile_rows(pkg, dev, M, N, fmt):
 
 @pytest.mark.parametrize("xdt,sdt,G", [("f16", np.float16, 128), ("bf16", "bf16", 32),
                                        ("f16", np.float32, 64)])
-@pytest.mark.parametrize("M,N,K", [(9, 2048, 4096), (16, 72, 96), (17, 264, 256), (33, 128, 1024),
-                                   (70, 768, 2048)])
+@pytest.mark.parametrize("M,N,K", [(9, 2048, 4096), (150, 72, 2048), (17, 264, 2048),
+                                   (90, 128, 2048), (33, 2656, 96), (70, 768, 2048)])
 def test_linear_awq_rows(pkg, dev, M, N, K, xdt, sdt, G):
     """Several rows on AutoAWQ weights in place run on MFMA: ragged row blocks, columns that
     end inside a 128-column strip, fewer steps of 32 than waves, K split or not; with the
