@@ -198,6 +198,10 @@ int    i4_linear(const void* x, int x_dtype, int M, const i4_qweight* w,
                  const void* bias, void* y, int y_dtype,
                  void* workspace, size_t workspace_bytes, hipStream_t stream);
 size_t i4_linear_workspace_bytes(const i4_qweight* w, int M);
+/* 1 when M rows of this AWQ weight run on MFMA (given the workspace), 0 when they run
+ * the GEMV: the MFMA path uses the workspace within the call only, while the GEMV
+ * keeps its status word there. */
+int    i4_linear_awq_mfma(const i4_qweight* w, int M);
 
 /* y = W RMSNorm(x) (+ bias) for every row of x in one launch: the decoder's
  * input_layernorm in front of the fused q|k|v projection (transformers

@@ -87,6 +87,7 @@ SIGNATURES = {
     "i4_linear": (c_int, [c_void_p, c_int, c_int, POINTER(QWeightC), c_void_p, c_void_p, c_int,
                           c_void_p, c_size_t, c_void_p]),
     "i4_linear_workspace_bytes": (c_size_t, [POINTER(QWeightC), c_int]),
+    "i4_linear_awq_mfma": (c_int, [POINTER(QWeightC), c_int]),
     "i4_unpack": (c_int, [POINTER(QWeightC), c_void_p, c_void_p]),
     "i4_dequant": (c_int, [POINTER(QWeightC), c_void_p, c_int, c_void_p]),
     "i4_repack_awq_to_ct": (c_int, [POINTER(QWeightC), c_void_p, c_void_p, c_void_p, c_int, c_int,

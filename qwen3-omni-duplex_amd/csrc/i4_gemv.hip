@@ -818,12 +818,20 @@ static bool awq_use_mm(const i4_qweight& w, int M) {
   const int slice = 16 * p.nwave * p.ppt;
   return M * p.P >= 112 || work >= (int64_t)(slice == 128 ? 24 : slice == 64 ? 12 : 8) << 20;
 }
-// Its fp32 partials stay clear of the split-K GEMV's (value, tag) pairs, whose tags must
-// not be met by chance, so that one workspace serves calls of any number of rows.
-static constexpr size_t MM_OFFSET = SK_HEAD + kSplitBytes;
+// Where its fp32 partials start in the workspace: behind the (value, tag) pairs of the rows
+// that this weight leaves to the split-K GEMV, whose tags must not be met by chance, so that
+// one workspace serves calls of any number of rows (and always behind the status word).
+static size_t awq_mm_offset(const i4_qweight& w) {
+  size_t o = SK_HEAD;
+  for (int r = 1; r <= kSplitRows; ++r) {
+    const size_t b = awq_use_mm(w, r) ? 0 : awq_split_bytes(awq_split_plan(w, r), r);
+    if (b > o) o = b;
+  }
+  return (o + 255) & ~(size_t)255;
+}
 static size_t awq_mm_bytes(const i4_qweight& w, int M) {
   const int ks = awq_mm_ksplit(M, w.N, w.K);
-  return ks > 1 ? MM_OFFSET + (size_t)ks * M * w.N * sizeof(float) : 0;
+  return ks > 1 ? awq_mm_offset(w) + (size_t)ks * M * w.N * sizeof(float) : 0;
 }
 
 // the tag of one call of the split-K GEMV: a process-wide count, never 0
@@ -959,6 +967,13 @@ size_t i4_linear_workspace_bytes(const i4_qweight* w, int M) {
   return i4_dq_gemv_workspace_bytes(w, M);
 }
 
+int i4_linear_awq_mfma(const i4_qweight* w, int M) {
+  i4_qweight nw;
+  if (!w || i4_check_weight(w, &nw) != I4_OK || nw.layout != I4_LAYOUT_AWQ) return 0;
+  nw.E = 1;
+  return awq_use_mm(nw, M);
+}
+
 int i4_linear(const void* x, int x_dtype, int M, const i4_qweight* w, const void* bias, void* y,
               int y_dtype, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   i4_qweight nw;
@@ -989,7 +1004,7 @@ int i4_linear(const void* x, int x_dtype, int M, const i4_qweight* w, const void
     const size_t need = awq_mm_bytes(nw, M);
     // without the workspace the GEMV runs, as for every number of rows
     if (!need || (workspace && workspace_bytes >= need && !((uintptr_t)workspace & 255))) {
-      float* part = need ? (float*)((char*)workspace + MM_OFFSET) : nullptr;
+      float* part = need ? (float*)((char*)workspace + awq_mm_offset(nw)) : nullptr;
 #define I4_MM_DT(XT_, ST_)                               \
   if (x_dtype == XT_ && nw.scale_dtype == ST_)           \
     return launch_awq_mm<XT_, ST_>(x, M, nw, bias, y, y_dtype, part, stream);

@@ -141,9 +141,8 @@ def linear(x: torch.Tensor, w: QWeight, bias: torch.Tensor | None = None,
     lb = _lib.lib()
     cw = w.c()
     nbytes = lb.i4_linear_workspace_bytes(ctypes.byref(cw), M)
-    # (the GEMV splits K for at most 8 rows)
-    if w.layout == "awq" and nbytes and (
-            M > 8 or nbytes != lb.i4_dq_gemv_workspace_bytes(ctypes.byref(cw), M)):
+    if w.layout == "awq" and nbytes and (M > 8  # the GEMV splits K for at most 8 rows
+                                         or lb.i4_linear_awq_mfma(ctypes.byref(cw), M)):
         # several rows on MFMA: the partial sums live from one launch of the call to the next
         # only, so they take memory of the call's stream (or graph) and not the kept
         # workspace, which other streams and captured calls of fewer rows may be using

@@ -55,15 +55,11 @@ def test_rows_leave_the_kept_workspace_alone(pkg, stub):
     assert stub.calls[-1][1] == lo
 
 
-def _mm_rows(pkg, N, K, G, rows, E=1):
-    """Which of the row counts take partials of the MFMA path (and not the GEMV's workspace)."""
+def _mm_rows(pkg, N, K, G, rows):
     import ctypes
 
     w = awq_linear(pkg, N, K, G).w.c()
-    lb = pkg.lib()
-    size = lambda M: lb.i4_linear_workspace_bytes(ctypes.byref(w), M)
-    return [M for M in rows if size(M) and size(M) != lb.i4_dq_gemv_workspace_bytes(
-        ctypes.byref(w), M)]
+    return [M for M in rows if pkg.lib().i4_linear_awq_mfma(ctypes.byref(w), M)]
 
 
 @pytest.mark.parametrize("N,K,G,first", [
@@ -85,3 +81,19 @@ def test_rows_take_mfma_where_it_was_measured_faster(pkg, N, K, G, first):
         few, many = [r for r in rows if r <= 8], [r for r in rows if r > 8]
         for part, last in ((few, 8), (many, 159)):
             assert not part or part == list(range(part[0], last + 1))
+
+
+@pytest.mark.parametrize("N,K,M,gemv_rows,ksplit", [
+    (2048, 4096, 24, 3, 16), (512, 2048, 24, 6, 16), (4096, 2048, 33, 3, 4),
+    (2048, 256, 64, 5, 2), (768, 768, 24, 8, 6),
+])
+def test_partials_start_behind_the_weights_own_pairs(pkg, N, K, M, gemv_rows, ksplit):
+    """The workspace of M rows: what the split GEMV of up to gemv_rows rows of this weight
+    uses (at least the 256-byte header), then ksplit partials of M x N fp32."""
+    import ctypes
+
+    w = awq_linear(pkg, N, K).w.c()
+    lb = pkg.lib()
+    head = max([256] + [lb.i4_dq_gemv_workspace_bytes(ctypes.byref(w), r)
+                        for r in range(1, gemv_rows + 1)])
+    assert lb.i4_linear_workspace_bytes(ctypes.byref(w), M) == head + ksplit * M * N * 4
