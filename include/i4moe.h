@@ -279,7 +279,9 @@ int    i4_moe_forward(const void* x, int x_dtype, int T, const i4_moe_weights* w
  * tagged with it and which a later launch of the call advances, so no word left by
  * an earlier call can pass for this call's; any starting value works (no
  * initialisation; a word left by something else passes with odds 2^-32).  Calls
- * that share one workspace must not overlap. */
+ * that share one workspace must not overlap.  More than 1024 tokens run in passes
+ * of up to 4096, where the shape has tiles for it, given the workspace named here;
+ * with less, down to that of 1024 tokens, in passes of 1024. */
 size_t i4_moe_workspace_bytes(int T, int H, int I, int E, int topk);
 
 /* i4_moe_forward for 2 <= T <= 64 tokens with the bound of its in-launch wait set by
@@ -310,7 +312,8 @@ int    i4_moe_forward_bounded(const void* x, int x_dtype, int T, const i4_moe_we
  * projections, gave up waiting for the activations of its own launch (its output
  * rows are then NaN), or a ranking wave of the 2..64-token routing launch (router
  * logits and top-k in one launch, E <= 128) gave up waiting for its token's logits
- * (its routing weights, and so its output row, are then NaN).  The host reads it after the stream has finished the call; a
+ * (its routing weights, and so its output row, are then NaN).  It lies at the same
+ * offset for all sizes.  The host reads it after the stream has finished the call; a
  * stack call reports a give-up in any of its layers.  The wait only ends that
  * way if the launch's workgroups are not dispatched in block order, which the
  * wait assumes (no reference counterpart: the reference faults instead,

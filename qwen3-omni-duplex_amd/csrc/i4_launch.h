@@ -64,4 +64,6 @@ int moe_forward_status(const void* x, int x_dtype, int T, const i4_moe_weights* 
                        int topk, int renorm, const void* logits, const void* residual, void* out,
                        int32_t* sel_out, float* w_out, void* workspace, size_t workspace_bytes,
                        int32_t* status, hipStream_t stream);
+// the workspace below which i4_moe_forward refuses a call: passes of at most 1024 tokens
+size_t moe_least_workspace(int T, int H, int I, int E, int topk);
 }  // namespace i4

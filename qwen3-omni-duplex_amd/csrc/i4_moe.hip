@@ -297,9 +297,6 @@ inline size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
 inline bool tile_gemm_fits(int H, int I, int E, int topk) {
   return I % (16 * TG_NW) == 0 && H % (32 * TG_NW) == 0 && TCHUNK * topk >= 64 * E;
 }
-inline int tokens_per_pass(int H, int I, int E, int topk) {
-  return tile_gemm_fits(H, I, E, topk) ? BIG_CHUNK : TCHUNK;
-}
 
 struct MoeWs {
   void* logits;
@@ -318,8 +315,10 @@ struct MoeWs {
   size_t bytes;
 };
 
-MoeWs carve(void* base, int T, int H, int I, int E, int topk) {
-  const int tc = tokens_per_pass(H, I, E, topk), Tc = T < tc ? T : tc;
+// The workspace of a call in passes of at most tc tokens.  The epoch and the status word come
+// first: they lie at the same offsets for every T and tc.
+MoeWs carve(void* base, int T, int H, int I, int E, int topk, int tc) {
+  const int Tc = T < tc ? T : tc;
   const size_t Tk = (size_t)Tc * topk;
   MoeWs m;
   size_t o = 0;
@@ -331,6 +330,7 @@ MoeWs carve(void* base, int T, int H, int I, int E, int topk) {
   // the tag epoch of the fused routing's words first, at the same offset for every T, so
   // that no other layout of the workspace writes over it
   m.epoch = (u32*)take(4);
+  m.status = (int32_t*)take(4);
   // [Tc][E] half logits, or [Tc][E / 2] (value pair, tag) words of the fused routing
   m.logits = take((size_t)Tc * E * 4);
   m.xn = (uint16_t*)take((size_t)Tc * H * 2);
@@ -343,9 +343,18 @@ MoeWs carve(void* base, int T, int H, int I, int E, int topk) {
   m.n_entries = (int*)take(4);
   m.mf_entries = (int4*)take((E + Tk / MF_TOK + 1) * sizeof(int4));
   m.n_mf_entries = (int*)take(4);
-  m.status = (int32_t*)take(4);
   m.bytes = o;
   return m;
+}
+
+// Tokens per pass: the 128-token tiles' passes need a workspace of their own size, so a
+// smaller one (the library's static scratch, one that a caller sized for 1024 tokens) is
+// served in passes of TCHUNK as any call of 1024 tokens is.
+int tokens_per_pass(int T, int H, int I, int E, int topk, size_t bytes) {
+  return T > TCHUNK && tile_gemm_fits(H, I, E, topk) &&
+                 carve(nullptr, T, H, I, E, topk, BIG_CHUNK).bytes <= bytes
+             ? BIG_CHUNK
+             : TCHUNK;
 }
 
 TW to_tw(const i4_qweight& w) {
@@ -616,12 +625,11 @@ int moe_forward_impl(const void* x, int x_dtype, int T, const i4_moe_weights* we
   if (((uintptr_t)x & 15) || ((uintptr_t)out & 15) || ((uintptr_t)residual & 15))
     return I4_ERR_ALIGN;
   const int H = gu.K, I = dn.K, E = gu.E;
-  const MoeWs need = carve(nullptr, T, H, I, E, topk);
-  if (!workspace || workspace_bytes < need.bytes) return I4_ERR_WORKSPACE;
+  const int tc = tokens_per_pass(T, H, I, E, topk, workspace_bytes);
+  MoeWs ws = carve(workspace, T, H, I, E, topk, tc);
+  if (!workspace || workspace_bytes < ws.bytes) return I4_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255) return I4_ERR_ALIGN;
-  MoeWs ws = carve(workspace, T, H, I, E, topk);
   if (status) ws.status = status;  // the caller's status word instead of the workspace's
-  const int tc = tokens_per_pass(H, I, E, topk);
   for (int t0 = 0; t0 < T; t0 += tc) {
     const int Tc = T - t0 < tc ? T - t0 : tc;
     const char* xs = (const char*)x + (size_t)t0 * H * 2;
@@ -651,11 +659,11 @@ int moe_decode_bufs(const i4_moe_weights* mw, int x_dtype, int topk, void* ws, s
   const int H = gu.K, I = dn.K, E = gu.E;
   if ((H != 1024 && H != 2048) || !moe_m1_ct_fits(topk, H, I)) return I4_ERR_SHAPE;
   if (((uintptr_t)mw->router_w & 15) || ((uintptr_t)mw->norm_w & 15)) return I4_ERR_ALIGN;
-  if (!ws || ws_bytes < carve(nullptr, 1, H, I, E, topk).bytes) return I4_ERR_WORKSPACE;
+  if (!ws || ws_bytes < carve(nullptr, 1, H, I, E, topk, TCHUNK).bytes) return I4_ERR_WORKSPACE;
   if ((uintptr_t)ws & 255) return I4_ERR_ALIGN;
   MoeOps ops;
   if (!pick_ops(x_dtype, gu.scale_dtype, dn.scale_dtype, &ops)) return I4_ERR_DTYPE;
-  const MoeWs w = carve(ws, 1, H, I, E, topk);
+  const MoeWs w = carve(ws, 1, H, I, E, topk, TCHUNK);
   b->logits = (uint16_t*)w.logits;
   b->xn = w.xn;
   b->act = (u32x4*)w.act;
@@ -674,7 +682,7 @@ int moe_decode_experts(const MoeDecodeBufs& b, int x_dtype, int topk, int renorm
                        const void* residual, void* out, void* ws, hipStream_t s) {
   const i4_qweight& gu = b.gate_up;
   const i4_qweight& dn = b.down;
-  const MoeWs w = carve(ws, 1, gu.K, dn.K, gu.E, topk);
+  const MoeWs w = carve(ws, 1, gu.K, dn.K, gu.E, topk, TCHUNK);
   MoeOps ops;
   if (!pick_ops(x_dtype, gu.scale_dtype, dn.scale_dtype, &ops)) return I4_ERR_DTYPE;
   // the status word was reset before the router launch, which may have reported in it
@@ -688,11 +696,15 @@ int moe_decode_experts_x(const MoeDecodeBufs& b, int x_dtype, int topk, int reno
   const i4_qweight& gu = b.gate_up;
   const i4_qweight& dn = b.down;
   if (!moe_m1x_ct_fits(topk, gu.K, dn.K)) return I4_ERR_SHAPE;
-  const MoeWs w = carve(ws, 1, gu.K, dn.K, gu.E, topk);
+  const MoeWs w = carve(ws, 1, gu.K, dn.K, gu.E, topk, TCHUNK);
   MoeOps ops;
   if (!pick_ops(x_dtype, gu.scale_dtype, dn.scale_dtype, &ops)) return I4_ERR_DTYPE;
   const GateUpArgs a{true, topk, topk, gu.E, renorm, w.xn, w.sel, w.logits, w.w, w.act, nullptr};
   return ops.moe_m1x_ct(a, to_tw(gu), to_tw(dn), ypart, w.status, kHandoffPolls, false, s);
+}
+
+size_t moe_least_workspace(int T, int H, int I, int E, int topk) {
+  return carve(nullptr, T, H, I, E, topk, TCHUNK).bytes;
 }
 
 int moe_forward_status(const void* x, int x_dtype, int T, const i4_moe_weights* weights,
@@ -802,13 +814,13 @@ extern "C" {
 
 size_t i4_moe_workspace_bytes(int T, int H, int I, int E, int topk) {
   if (T < 1 || H < 1 || I < 1 || E < 1 || topk < 1) return 0;
-  return carve(nullptr, T, H, I, E, topk).bytes;
+  return carve(nullptr, T, H, I, E, topk, tokens_per_pass(T, H, I, E, topk, SIZE_MAX)).bytes;
 }
 
 size_t i4_moe_status_offset(int T, int H, int I, int E, int topk) {
   if (T < 1 || H < 1 || I < 1 || E < 1 || topk < 1) return 0;
   char* const base = (char*)(uintptr_t)4096;  // carve() lays out from any aligned base
-  return (size_t)((char*)carve(base, T, H, I, E, topk).status - base);
+  return (size_t)((char*)carve(base, T, H, I, E, topk, TCHUNK).status - base);
 }
 
 int i4_moe_forward(const void* x, int x_dtype, int T, const i4_moe_weights* weights, int topk,
@@ -935,14 +947,15 @@ int i4_moe_stack_forward(const void* x, int x_dtype, int T, const i4_moe_weights
   for (int l = 1; l < n_layers; ++l)
     if (layers[l].gate_up.K != H || layers[l].down.K != I || layers[l].gate_up.E != E)
       return I4_ERR_SHAPE;
-  const size_t mbytes = i4_moe_workspace_bytes(T, H, I, E, topk);
-  if (!workspace || workspace_bytes < mbytes + stack_extra_bytes(T, H, topk))
-    return I4_ERR_WORKSPACE;
+  const size_t extra = stack_extra_bytes(T, H, topk);
+  size_t mbytes = i4_moe_workspace_bytes(T, H, I, E, topk);
+  if (workspace_bytes < mbytes + extra) mbytes = i4::moe_least_workspace(T, H, I, E, topk);
+  if (!workspace || workspace_bytes < mbytes + extra) return I4_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255) return I4_ERR_ALIGN;
   void* buf = (char*)workspace + mbytes;
   if (T == 1 && stack_xcd_local(layers, n_layers, x_dtype, topk))
     return stack_m1x(x, x_dtype, layers, n_layers, topk, renorm, out,
-                     carve(workspace, 1, H, I, E, topk), (uint16_t*)buf,
+                     carve(workspace, 1, H, I, E, topk, TCHUNK), (uint16_t*)buf,
                      (uint16_t*)((char*)buf + al256((size_t)H * 2)),
                      (uint16_t*)((char*)buf + 2 * al256((size_t)H * 2)), stream);
   const void* h = x;
@@ -966,10 +979,10 @@ int i4_moe_route_sum(const void* res, int x_dtype, const void* ypart,
   if (!res || (ypart && !h_out)) return I4_ERR_NULL;
   if (((uintptr_t)res & 15) || ((uintptr_t)ypart & 15) || ((uintptr_t)h_out & 15))
     return I4_ERR_ALIGN;
-  if (!workspace || workspace_bytes < carve(nullptr, 1, b.H, b.I, b.E, topk).bytes)
+  if (!workspace || workspace_bytes < carve(nullptr, 1, b.H, b.I, b.E, topk, TCHUNK).bytes)
     return I4_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255) return I4_ERR_ALIGN;
-  const MoeWs ws = carve(workspace, 1, b.H, b.I, b.E, topk);
+  const MoeWs ws = carve(workspace, 1, b.H, b.I, b.E, topk, TCHUNK);
   return x_route(res, x_dtype, ypart, weights, b, topk, h_out, ws, reset_status != 0, stream);
 }
 
@@ -982,10 +995,10 @@ int i4_moe_experts_x(const void* h, int x_dtype, const i4_moe_weights* weights, 
   if (!ypart || (!weights->norm_w && !h)) return I4_ERR_NULL;
   if (((uintptr_t)ypart & 15) || ((uintptr_t)h & 15)) return I4_ERR_ALIGN;
   if (max_polls < 0) return I4_ERR_SHAPE;
-  if (!workspace || workspace_bytes < carve(nullptr, 1, b.H, b.I, b.E, topk).bytes)
+  if (!workspace || workspace_bytes < carve(nullptr, 1, b.H, b.I, b.E, topk, TCHUNK).bytes)
     return I4_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255) return I4_ERR_ALIGN;
-  const MoeWs ws = carve(workspace, 1, b.H, b.I, b.E, topk);
+  const MoeWs ws = carve(workspace, 1, b.H, b.I, b.E, topk, TCHUNK);
   return x_experts(h, weights, b, topk, renorm, ypart, ws, max_polls, down_only != 0, stream);
 }
 
@@ -998,10 +1011,10 @@ int i4_moe_sum(const void* res, int x_dtype, const void* ypart, const i4_moe_wei
   if (!res || !ypart || !out) return I4_ERR_NULL;
   if (((uintptr_t)res & 15) || ((uintptr_t)ypart & 15) || ((uintptr_t)out & 15))
     return I4_ERR_ALIGN;
-  if (!workspace || workspace_bytes < carve(nullptr, 1, b.H, b.I, b.E, topk).bytes)
+  if (!workspace || workspace_bytes < carve(nullptr, 1, b.H, b.I, b.E, topk, TCHUNK).bytes)
     return I4_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255) return I4_ERR_ALIGN;
-  const MoeWs ws = carve(const_cast<void*>(workspace), 1, b.H, b.I, b.E, topk);
+  const MoeWs ws = carve(const_cast<void*>(workspace), 1, b.H, b.I, b.E, topk, TCHUNK);
   return i4_launch_moe_sum(res, ypart, ws.w, topk, x_dtype, b.H, out, stream);
 }
 

@@ -53,9 +53,9 @@ int i4_moe_forward_noalloc(const void* x, int x_dtype, int T, const i4_moe_weigh
                            void* out, int32_t* sel_out, float* w_out, int32_t* status_out,
                            hipStream_t stream) {
   if (!weights) return I4_ERR_NULL;
-  const size_t need = i4_moe_workspace_bytes(T, weights->gate_up.K, weights->down.K,
-                                             weights->gate_up.E, topk);
-  if (need == 0) return I4_ERR_SHAPE;
+  const int H = weights->gate_up.K, I = weights->down.K, E = weights->gate_up.E;
+  if (i4_moe_workspace_bytes(T, H, I, E, topk) == 0) return I4_ERR_SHAPE;
+  const size_t need = i4::moe_least_workspace(T, H, I, E, topk);
   if (need > (size_t)I4_NOALLOC_SCRATCH_BYTES) return I4_ERR_SCRATCH;
   int dev = -1;
   if (stream) {

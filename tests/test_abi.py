@@ -502,3 +502,30 @@ def test_down_wait_validation_codes(pkg):
     tile = _qw(_lib, E=128, N=2048, K=768, group=128, layout=2)
     assert lib.i4_moe_down_wait(0x30000, 1, ctypes.byref(tile), 0x40000, 128, 8, 1, None, 0x50000,
                                 0x60000, 16, None) == -5
+
+
+def test_status_word_has_one_place(pkg):
+    """Whatever the sizes and the passes of a call, so a workspace that served several kinds
+    of calls has one status word."""
+    lib = pkg.lib()
+    offs = {lib.i4_moe_status_offset(*a) for a in ((1, 2048, 768, 128, 8), (64, 2048, 768, 128, 8),
+                                                   (1024, 256, 128, 24, 8), (5000, 1024, 384, 64, 6))}
+    assert len(offs) == 1
+
+
+def test_noalloc_serves_many_tokens_of_a_small_block(pkg):
+    """A block whose passes of 1024 tokens fit the static scratch is served for any number of
+    tokens.  x is NULL, so nothing runs: without a GPU the scratch's address is refused (-8),
+    with one the pointer (-1); -11 would be the scratch limit."""
+    from qwen3_omni_duplex_amd import _lib
+
+    lib = pkg.lib()
+    H, I, E, k = 256, 128, 24, 8
+    tile = lambda N, K: _qw(_lib, layout=2, E=E, N=N, K=K, group=32)
+    mw = _lib.MoeWeightsC(gate_up=tile(2 * I, H), down=tile(H, I), router_w=0x70000)
+    small = lib.i4_moe_workspace_bytes(1024, H, I, E, k)
+    assert small < (8 << 20) < lib.i4_moe_workspace_bytes(2000, H, I, E, k)
+    for T in (1024, 1025, 2000, 4096, 20000):
+        rc = lib.i4_moe_forward_noalloc(None, 2, T, ctypes.byref(mw), k, 1, None, None, 0x50000,
+                                        None, None, None, None)
+        assert rc in (-8, -1), (T, rc)

@@ -60,3 +60,34 @@ def test_noalloc_logits_and_norm(pkg, dev):
         got = pkg.moe_forward_noalloc(x, moe.gate_up, moe.down, K8, router_w=moe.router_w,
                                       norm_w=nw, residual=x, **tiles)
         assert torch.equal(got, want)
+
+
+def test_noalloc_many_tokens_of_a_small_block(pkg, dev):
+    """A block small enough for passes of 1024 tokens in the scratch takes any number of tokens,
+    as i4_moe_forward does with the workspace of 1024 tokens: the same result bit for bit."""
+    import ctypes
+
+    rng = np.random.default_rng(203)
+    h, i, e = 256, 128, 24
+    moe, _, _, _ = _awq_moe(pkg, dev, rng, E=e, H=h, I=i, G=32)
+    tiles = dict(gate_up_tile=moe.gate_up_tile, down_tile=moe.down_tile)
+    lib = pkg.lib()
+    nbytes = lib.i4_moe_workspace_bytes(1024, h, i, e, K8)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    mw = pkg.ops.moe_weights_c(moe.gate_up, moe.down, moe.router_w, None, 1e-6, **tiles)
+    for T in (1300, 2500):
+        assert lib.i4_moe_workspace_bytes(T, h, i, e, K8) > (8 << 20)
+        x = t_(make_x(rng, (T, h), "f16"), dev)
+        want = torch.empty_like(x)
+        call = lambda n: lib.i4_moe_forward(
+            x.data_ptr(), 1, T, ctypes.byref(mw), K8, 1, None, x.data_ptr(), want.data_ptr(),
+            None, None, ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream)
+        assert call(nbytes - 1) == -7
+        assert call(nbytes) == 0
+        got = pkg.moe_forward_noalloc(x, moe.gate_up, moe.down, K8, router_w=moe.router_w,
+                                      residual=x, **tiles)
+        assert torch.isfinite(want).all() and torch.equal(got, want)
+        # and what the 4096-token passes give, up to the two tile sizes' rounding of scales
+        big = pkg.moe_forward(x, moe.gate_up, moe.down, K8, router_w=moe.router_w, residual=x,
+                              **tiles)
+        assert (big - want).abs().max() <= 2e-3 * want.abs().max()
