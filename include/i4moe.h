@@ -283,6 +283,12 @@ int    i4_moe_forward(const void* x, int x_dtype, int T, const i4_moe_weights* w
  * of up to 4096, where the shape has tiles for it, given the workspace named here;
  * with less, down to that of 1024 tokens, in passes of 1024. */
 size_t i4_moe_workspace_bytes(int T, int H, int I, int E, int topk);
+/* i4_moe_forward with its status word at `status` (int32, device) instead of in the
+ * workspace, for callers whose workspace lives for one call only. */
+int    i4_moe_forward_status(const void* x, int x_dtype, int T, const i4_moe_weights* weights,
+                             int topk, int renorm, const void* logits, const void* residual,
+                             void* out, int32_t* sel_out, float* w_out, void* workspace,
+                             size_t workspace_bytes, int32_t* status, hipStream_t stream);
 
 /* i4_moe_forward for 2 <= T <= 64 tokens with the bound of its in-launch wait set by
  * the caller (no reference counterpart: the reference runs the two projections as

@@ -102,6 +102,9 @@ SIGNATURES = {
                                c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                c_size_t, c_void_p]),
     "i4_moe_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "i4_moe_forward_status": (c_int, [c_void_p, c_int, c_int, POINTER(MoeWeightsC), c_int,
+                                      c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                      c_void_p, c_size_t, c_void_p, c_void_p]),
     "i4_moe_forward_bounded": (c_int, [c_void_p, c_int, c_int, POINTER(MoeWeightsC), c_int,
                                        c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t,
                                        c_int, c_int, c_void_p]),

@@ -831,6 +831,15 @@ int i4_moe_forward(const void* x, int x_dtype, int T, const i4_moe_weights* weig
                           w_out, workspace, workspace_bytes, true, stream);
 }
 
+int i4_moe_forward_status(const void* x, int x_dtype, int T, const i4_moe_weights* weights,
+                          int topk, int renorm, const void* logits, const void* residual,
+                          void* out, int32_t* sel_out, float* w_out, void* workspace,
+                          size_t workspace_bytes, int32_t* status, hipStream_t stream) {
+  if (!status) return I4_ERR_NULL;
+  return i4::moe_forward_status(x, x_dtype, T, weights, topk, renorm, logits, residual, out,
+                                sel_out, w_out, workspace, workspace_bytes, status, stream);
+}
+
 int i4_moe_forward_bounded(const void* x, int x_dtype, int T, const i4_moe_weights* weights,
                            int topk, int renorm, const void* logits, const void* residual,
                            void* out, void* workspace, size_t workspace_bytes, int max_polls,

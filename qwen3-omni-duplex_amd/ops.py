@@ -353,8 +353,20 @@ def moe_forward(x: torch.Tensor, gate_up: QWeight, down: QWeight, top_k: int,
     wts = torch.empty(T, top_k, dtype=torch.float32, device=dev) if return_routing else None
     lb = _lib.lib()
     nbytes = lb.i4_moe_workspace_bytes(T, H, I, E, top_k)
-    ws = (workspace or Workspace()).get(nbytes, dev)
+    kept = workspace or Workspace()
     mw = moe_weights_c(gate_up, down, router_w, norm_w, norm_eps, gate_up_tile, down_tile)
+    if T > 1024 and nbytes > lb.i4_moe_workspace_bytes(1024, H, I, E, top_k):
+        # passes of up to 4096 tokens: their scratch (204 MB at H 2048, FFN 768, top-8) is
+        # memory of this call, which the layers of a model take one after the other; the
+        # workspace keeps the status word alone
+        off = lb.i4_moe_status_offset(T, H, I, E, top_k)
+        ws, status = torch.empty(nbytes, dtype=torch.uint8, device=dev), kept.get(off + 4, dev)
+        _lib.check(lb.i4_moe_forward_status(
+            xf.data_ptr(), xt, T, ctypes.byref(mw), top_k, int(norm_topk_prob), _lib.ptr(lg),
+            _lib.ptr(rs), out.data_ptr(), _lib.ptr(sel), _lib.ptr(wts), ws.data_ptr(), nbytes,
+            status.data_ptr() + off, _lib.stream(dev)))
+        return (out.view(shape), sel, wts) if return_routing else out.view(shape)
+    ws = kept.get(nbytes, dev)
     if _bounded is not None:
         _lib.check(lb.i4_moe_forward_bounded(
             xf.data_ptr(), xt, T, ctypes.byref(mw), top_k, int(norm_topk_prob), _lib.ptr(lg),

@@ -62,3 +62,14 @@ def test_awq_linear_graph_after_larger_calls(pkg, dev, rows, N, K):
     larger = [t_(make_x(rng, (n, K), "f16"), dev) for n in (24, 256)]
     replay_after_larger(lin, small, larger, lin.workspace)
     assert pkg.ops.gemv_status(lin.workspace) == 0
+
+
+def test_moe_prompt_after_capture(pkg, dev):
+    """A captured call of 70 tokens, then prompts beyond 1024: the workspace stays."""
+    rng = np.random.default_rng(73)
+    moe, _, _, _ = _awq_moe(pkg, dev, rng, E=24, H=256, I=128, G=32)
+    small = [t_(make_x(rng, (70, 256), "f16"), dev) for _ in range(3)]
+    larger = [t_(make_x(rng, (n, 256), "f16"), dev) for n in (1500, 4100)]
+    replay_after_larger(moe, small, larger, moe.workspace)
+    assert moe.workspace.buf.numel() == pkg.lib().i4_moe_workspace_bytes(70, 256, 128, 24, 8)
+    assert pkg.moe_status(moe.workspace, 4100, 256, 128, 24, 8) == 0
