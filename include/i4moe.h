@@ -622,6 +622,9 @@ int    i4_dmoe_forward(const void* x, int x_dtype, int T, const i4_dmoe_weights*
  * grouping and the fp32 slot outputs of up to 1024 tokens; 16-byte aligned, no
  * initial contents).  Calls sharing one workspace must not overlap. */
 size_t i4_dmoe_workspace_bytes(int T, int E, int topk, int I, int Is);
+/* The same for hidden size H: i4_dmoe_workspace_bytes does not know it and names what
+ * the largest (2048) needs. */
+size_t i4_dmoe_workspace_bytes_h(int T, int E, int topk, int H, int I, int Is);
 
 /* One decode token (T = 1) with router_w in the block and 16-bit routed experts
  * runs in two launches:

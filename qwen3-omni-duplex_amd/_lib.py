@@ -167,6 +167,7 @@ SIGNATURES = {
                                 c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                 c_size_t, c_void_p]),
     "i4_dmoe_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
+    "i4_dmoe_workspace_bytes_h": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "i4_dmoe_status_offset": (c_size_t, [c_int, c_int, c_int, c_int, c_int]),
     "i4_dmoe_down_wait": (c_int, [c_void_p, c_int, POINTER(DmoeWeightsC), c_int, c_int,
                                   c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_int,

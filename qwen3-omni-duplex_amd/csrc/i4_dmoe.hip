@@ -389,7 +389,7 @@ struct DmoeWs {
 
 // act_s follows act directly: the router launch of a single-launch decode
 // marks both pending as one range
-DmoeWs dmoe_ws_layout(int T, int E, int topk, int I, int Is) {
+DmoeWs dmoe_ws_layout(int T, int E, int topk, int H, int I, int Is) {
   DmoeWs l;
   size_t o = 0;
   l.logits = o; o += align256((size_t)T * E * 2);
@@ -405,9 +405,8 @@ DmoeWs dmoe_ws_layout(int T, int E, int topk, int I, int Is) {
     l.perm = o;      o += align256((size_t)Tc * topk * 4);
     l.entries = o;   o += align256(dg_max_entries(Tc, E, topk) * sizeof(int4));
     l.n_entries = o; o += align256(4);
-    // fp32 slot outputs; the hidden size is not known here, so its limit
-    l.ys = o;        o += align256((size_t)Tc * topk * DMAX_H * 4);
-    l.ys_s = o;      o += align256(Is ? (size_t)Tc * DMAX_H * 4 : 0);
+    l.ys = o;        o += align256((size_t)Tc * topk * H * 4);  // fp32 slot outputs
+    l.ys_s = o;      o += align256(Is ? (size_t)Tc * H * 4 : 0);
   }
   l.total = o;
   return l;
@@ -464,7 +463,12 @@ int dmoe_launch(const DGateUpArgs& ga, const DDownArgs& da, int T, int H, const 
 
 extern "C" size_t i4_dmoe_workspace_bytes(int T, int E, int topk, int I, int Is) {
   if (T < 1 || E < 1 || topk < 1 || I < 0 || Is < 0) return 0;
-  return dmoe_ws_layout(T, E, topk, I, Is).total;
+  return dmoe_ws_layout(T, E, topk, DMAX_H, I, Is).total;
+}
+
+extern "C" size_t i4_dmoe_workspace_bytes_h(int T, int E, int topk, int H, int I, int Is) {
+  if (T < 1 || E < 1 || topk < 1 || H < 1 || H > DMAX_H || I < 0 || Is < 0) return 0;
+  return dmoe_ws_layout(T, E, topk, H, I, Is).total;
 }
 
 namespace {
@@ -510,7 +514,7 @@ int dmoe_impl(const void* x, int x_dtype, int T, const i4_dmoe_weights* wts, int
     return I4_ERR_ALIGN;
   const bool ri8 = gu.scale != nullptr, si8 = has_shared && wts->shared_gate_up.scale;
   if (stage_bytes(topk * I + Is, ri8 || si8) > 65536) return I4_ERR_SHAPE;
-  const DmoeWs l = dmoe_ws_layout(T, E, topk, I, Is);
+  const DmoeWs l = dmoe_ws_layout(T, E, topk, H, I, Is);
   if (!workspace || workspace_bytes < l.total) return I4_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 15) return I4_ERR_ALIGN;
   char* ws = (char*)workspace;
@@ -620,7 +624,7 @@ extern "C" int i4_dmoe_forward(const void* x, int x_dtype, int T, const i4_dmoe_
 
 extern "C" size_t i4_dmoe_status_offset(int T, int E, int topk, int I, int Is) {
   if (T < 1 || E < 1 || topk < 1 || I < 0 || Is < 0) return 0;
-  return dmoe_ws_layout(T, E, topk, I, Is).status;
+  return dmoe_ws_layout(T, E, topk, DMAX_H, I, Is).status;
 }
 
 extern "C" int i4_dmoe_down_wait(const void* x, int x_dtype, const i4_dmoe_weights* wts,

@@ -1015,7 +1015,7 @@ def dmoe_forward(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top
                              shared_gate_up, shared_down, shared_gate_w, shared_gate_up_scale,
                              shared_down_scale)
     lb = _lib.lib()
-    ws = (workspace or Workspace()).get(lb.i4_dmoe_workspace_bytes(T, E, top_k, I, Is), dev)
+    ws = (workspace or Workspace()).get(lb.i4_dmoe_workspace_bytes_h(T, E, top_k, H, I, Is), dev)
     _lib.check(lb.i4_dmoe_forward(xf.data_ptr(), xt, T, ctypes.byref(dw), top_k,
                                   int(norm_topk_prob), _lib.ptr(lg), _lib.ptr(rs),
                                   out.data_ptr(), _lib.ptr(sel), _lib.ptr(wts), ws.data_ptr(),

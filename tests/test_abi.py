@@ -529,3 +529,19 @@ def test_noalloc_serves_many_tokens_of_a_small_block(pkg):
         rc = lib.i4_moe_forward_noalloc(None, 2, T, ctypes.byref(mw), k, 1, None, None, 0x50000,
                                         None, None, None, None)
         assert rc in (-8, -1), (T, rc)
+
+
+def test_dense_moe_workspace_by_hidden_size(pkg):
+    """Beyond what the per-token kernels need, a grouped call holds the fp32 slot outputs of the
+    actual hidden size (plus the sorted pairs and entries, 16 bytes a pair at most)."""
+    lib = pkg.lib()
+    E, k, I, Is = 128, 6, 384, 768
+    for T, H in ((700, 1024), (700, 2048), (5000, 512)):
+        base = T * (2 * E + 8 * k + 4 + 2 * k * I + 2 * Is)
+        slots = min(T, 1024) * (k + 1) * H * 4
+        got = lib.i4_dmoe_workspace_bytes_h(T, E, k, H, I, Is)
+        assert base + slots <= got <= base + slots + 16 * (min(T, 1024) * k + E) + 13 * 256
+    assert lib.i4_dmoe_workspace_bytes_h(700, E, k, 2048, I, Is) == lib.i4_dmoe_workspace_bytes(
+        700, E, k, I, Is)
+    assert lib.i4_dmoe_workspace_bytes_h(1, E, k, 0, I, Is) == 0
+    assert lib.i4_dmoe_workspace_bytes_h(1, E, k, 2049, I, Is) == 0
