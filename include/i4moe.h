@@ -610,15 +610,16 @@ typedef struct i4_dmoe_weights {
  * rest is fp32 and the output is rounded once.  residual, sel_out and w_out
  * ([T][topk], fp32) are optional.  H % 16 == 0, 16 <= H <= 2048; I, Is multiples
  * of 16, at most 1024 (16-bit) or 2048 (int8); E <= 512; topk <= 8, <= 7 with a
- * shared expert; T <= 65535.  Calls of less than 12 tokens stream each token's own
- * experts' rows (decode-shaped; the reference gathers per token as well,
- * fused_moe.py:121); longer ones sort the tokens by expert and read an expert's rows once
- * for up to 64 of them.  A token's output is the same bit for bit either way. */
+ * shared expert; T <= 65535.  Calls of few tokens (less than 12 at the Talker's sizes, more
+ * where the experts are smaller) stream each token's own experts' rows (decode-shaped;
+ * the reference gathers per token as well, fused_moe.py:121); the others sort the tokens by
+ * expert and read an expert's rows once for up to 64 of them.  A token's output is the
+ * same bit for bit either way. */
 int    i4_dmoe_forward(const void* x, int x_dtype, int T, const i4_dmoe_weights* weights,
                        int topk, int renorm, const void* logits, const void* residual,
                        void* out, int32_t* sel_out, float* w_out, void* workspace,
                        size_t workspace_bytes, hipStream_t stream);
-/* Workspace of i4_dmoe_forward (logits, routing, activations; from 12 tokens also the
+/* Workspace of i4_dmoe_forward (logits, routing, activations; for a grouped call also the
  * grouping and the fp32 slot outputs of up to 1024 tokens; 16-byte aligned, no
  * initial contents).  Calls sharing one workspace must not overlap. */
 size_t i4_dmoe_workspace_bytes(int T, int E, int topk, int I, int Is);

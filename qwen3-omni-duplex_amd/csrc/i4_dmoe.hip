@@ -10,9 +10,9 @@
 // and down [E][H][I], either in the activation dtype or int8 with one scale per
 // output row (the q8 mode, fused_moe.py:84-94: value = q * scale).
 //
-// Decode-shaped, for calls of less than DG_MIN_T tokens (longer ones are grouped by
-// expert, i4_dmoe_group.hip): the T tokens of a call run in one launch per stage (grid
-// z / y), each token streaming its own experts' rows.
+// Decode-shaped, for calls of few tokens or small experts (dmoe_grouped; the others are
+// grouped by expert, i4_dmoe_group.hip): the T tokens of a call run in one launch per stage
+// (grid z / y), each token streaming its own experts' rows.
 //   k_d_gate_up  one workgroup per (block of rows of gate and up, slot, token);
 //                slot < topk is a routed expert, ranked from the logits by every
 //                wave itself (workgroup (0, 0, t) also stores token t's routing);
@@ -374,16 +374,25 @@ namespace {
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 constexpr int DMAX_H = 2048;  // hidden sizes served
-// Tokens from which a call runs grouped by expert (i4_dmoe_group.hip).  The grouped path
-// is six launches instead of three, which an eager caller pays on the host: 42-44 us a
-// call up to 16 tokens, against 32 us (up to 8 tokens), 44.4 (12) and 56 (16) per token
-// (bf16; int8 the same).  Above: 117 -> 67 us at 37 tokens, 417 -> 95 at 150, 1832 -> 231
-// at 700; int8 121 -> 59, 458 -> 105, 2051 -> 307.
+// Whether a call runs grouped by expert (i4_dmoe_group.hip).  The grouped path is six launches
+// instead of three, which an eager caller pays on the host (34-41 us a call against 23-30),
+// and per token next to nothing; the per-token kernels take about 0.1 us a slot and 2.4e-7 us
+// a multiply-add of every token on top (at least 0.3 us a token).  The line is where those
+// reach the grouped call's time, at least 12 tokens.  Measured over 19 blocks (4..512 experts,
+// top 1..8, H 256..2048, I 64..1024, shared expert or none), 9..192 tokens, bf16 and int8,
+// eager and in a graph: no grouped call over 5 % slower.  us, eager, per token / grouped,
+// bf16: 128 experts, top-6, H 1024, I 384, shared 768: 12 tokens 41 / 41, 24 72 / 51, 128
+// 348 / 83; 16 experts, top-2, H 512, I 256: 24 tokens 24 / 35, 128 84 / 35; 512 experts,
+// top-4, H 256, I 128, shared 128: 24 tokens 30 / 40, 128 105 / 68.
 constexpr int DG_MIN_T = 12;
+bool dmoe_grouped(int T, int topk, int H, int I, int Is) {
+  const double token_us = 0.1 * topk + 2.4e-7 * 3 * H * ((double)topk * I + Is);
+  return T >= DG_MIN_T && T * (token_us > 0.3 ? token_us : 0.3) >= 34;
+}
 
 struct DmoeWs {
   size_t logits, sel, wts, sg, status, act, act_s;
-  size_t perm, entries, n_entries, ys, ys_s;  // the grouped path (T >= DG_MIN_T)
+  size_t perm, entries, n_entries, ys, ys_s;  // the grouped path
   size_t total;
 };
 
@@ -400,7 +409,7 @@ DmoeWs dmoe_ws_layout(int T, int E, int topk, int H, int I, int Is) {
   l.act = o;    o += align256((size_t)T * topk * I * 2);
   l.act_s = o;  o += align256((size_t)T * Is * 2);
   l.perm = l.entries = l.n_entries = l.ys = l.ys_s = o;
-  if (T >= DG_MIN_T) {
+  if (dmoe_grouped(T, topk, H, I, Is)) {
     const int Tc = T < DG_CHUNK ? T : DG_CHUNK;
     l.perm = o;      o += align256((size_t)Tc * topk * 4);
     l.entries = o;   o += align256(dg_max_entries(Tc, E, topk) * sizeof(int4));
@@ -565,7 +574,7 @@ int dmoe_impl(const void* x, int x_dtype, int T, const i4_dmoe_weights* wts, int
   da.sdn = has_shared ? to_dw(wts->shared_down) : DW{nullptr, nullptr, 0, 0, 0};
   da.residual = (const uint16_t*)residual;
   da.out = (uint16_t*)out;
-  if (T >= DG_MIN_T && dg_formats(ri8, si8)) {
+  if (dmoe_grouped(T, topk, H, I, Is) && dg_formats(ri8, si8)) {
     rc = i4_launch_topk(lg, x_dtype, T, E, topk, renorm, ga.sel, ga.wts, nullptr, 0, stream);
     for (int t0 = 0; rc == I4_OK && t0 < T; t0 += DG_CHUNK) {
       DGCall c;

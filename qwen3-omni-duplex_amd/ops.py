@@ -985,7 +985,7 @@ def dmoe_forward(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, top
     logits, gate_up + SiLU + routing, down + combine); one token with router_w and 16-bit
     experts runs in two (router logits; gate_up and down in one launch, the down
     workgroups waiting for the activations: dmoe_status reports a wait that gave up);
-    12 tokens or more are grouped by expert, so that an expert's weights are read once
+    many tokens (from 12 at the Talker's sizes) are grouped by expert: its weights are read once
     for all of its tokens (six launches), with the same result bit for bit."""
     dev = _lib.require_device(x, gate_up, down, router_w, logits, shared_gate_up, shared_down,
                               shared_gate_w, residual)

@@ -545,3 +545,20 @@ def test_dense_moe_workspace_by_hidden_size(pkg):
         700, E, k, I, Is)
     assert lib.i4_dmoe_workspace_bytes_h(1, E, k, 0, I, Is) == 0
     assert lib.i4_dmoe_workspace_bytes_h(1, E, k, 2049, I, Is) == 0
+
+
+@pytest.mark.parametrize("shape,first", [
+    # (experts, top-k, H, I, Is): the first T of a grouped call
+    ((128, 6, 1024, 384, 768), 12), ((128, 7, 2048, 768, 768), 12), ((16, 2, 512, 256, 0), 88),
+    ((512, 4, 256, 128, 128), 66), ((32, 1, 1024, 384, 768), 36), ((16, 1, 256, 64, 0), 114),
+])
+def test_dense_moe_groups_where_it_was_measured_faster(pkg, shape, first):
+    """Small blocks run per token for longer: the grouped call's launches cost more than their
+    tokens.  Only a grouped call's workspace holds the fp32 slot outputs."""
+    lib = pkg.lib()
+    E, k, H, I, Is = shape
+    held = [lib.i4_dmoe_workspace_bytes_h(T, E, k, H, I, Is) for T in range(0, first + 2)]
+    steps = [b - a for a, b in zip(held[1:], held[2:])]  # steps[n]: from n + 1 to n + 2 tokens
+    slots = first * k * H * 4
+    assert steps[first - 2] > slots
+    assert all(s < slots // 2 for n, s in enumerate(steps) if n != first - 2)

@@ -348,13 +348,16 @@ def test_dmoe_tokens_are_independent(pkg, dev, T, q8):
     (12, dict()), (13, dict(q8=True)),                      # the smallest grouped calls
     (65, dict(skew=True)), (129, dict(skew=True, q8=True)),  # an expert of 64 tokens and more
     (1030, dict()),                                          # two passes over the tokens
-    (40, dict(H=256, E=16, I=48, Is=32)), (40, dict(H=256, E=16, I=48, Is=32, q8=True)),
+    (80, dict(H=256, E=16, I=48, Is=32)), (80, dict(H=256, E=16, I=48, Is=32, q8=True)),
     (33, dict(H=2048, E=8, I=1024, Is=1024)),                # the longest rows
     (33, dict(H=2048, E=8, I=2048, Is=2048, q8=True, shared_q8=True)),
-    (33, dict(H=528, E=20, I=272, Is=528, fp16=True)),       # rows that end inside a lane round
-    (33, dict(H=528, E=20, I=272, Is=528, q8=True, shared_q8=True)),
+    (37, dict(H=528, E=20, I=272, Is=528, fp16=True)),       # rows that end inside a lane round
+    (37, dict(H=528, E=20, I=272, Is=528, q8=True, shared_q8=True)),
     (20, dict(shared=False, top_k=8, residual=True)),
     (20, dict(shared_q8=True)),                              # served by the per-token kernels
+    (20, dict(renorm=False)), (20, dict(logits=True)),
+    (20, dict(renorm=False, logits=True, q8=True, residual=True)),
+    (20, dict(nonfinite=True)), (20, dict(nonfinite=True, q8=True)),
 ])
 def test_dmoe_grouped_equals_per_token(pkg, dev, T, case):
     """Calls grouped by expert give the per-token kernels' output (calls of at most 8
@@ -371,7 +374,13 @@ def test_dmoe_grouped_equals_per_token(pkg, dev, T, case):
     if case.get("skew"):  # every token selects expert 3
         x[:, 0] = 8.0
         rw[3, 0] = 4.0
-    kw = dict(router_w=rw)
+    if case.get("nonfinite"):  # in three tokens; the router ignores their columns
+        x[3, 5], x[9, 6], x[17, 7] = float("inf"), float("nan"), float("-inf")
+        rw[:, 5:8] = 0.0
+    kw = dict(router_w=rw, norm_topk_prob=case.get("renorm", True))
+    if case.get("logits") or case.get("nonfinite"):
+        kw["router_w"] = None
+    lg = pkg.router_logits(torch.nan_to_num(x, 0.0, 0.0, 0.0), rw)
     gu, dn = S["gu"], S["dn"]
     if case.get("q8"):
         gu, kw["gate_up_scale"] = pkg.quantize_q8(gu)
@@ -385,14 +394,28 @@ def test_dmoe_grouped_equals_per_token(pkg, dev, T, case):
 
     def call(a, b):
         return pkg.dmoe_forward(x[a:b].contiguous(), gu, dn, top_k, return_routing=True,
+                                logits=None if kw["router_w"] is not None else lg[a:b],
                                 residual=None if res is None else res[a:b].contiguous(), **kw)
 
+    # the whole call runs grouped, the calls of 8 tokens do not: only a grouped call's
+    # workspace holds the fp32 slot outputs
+    sizes = gu.shape[0], top_k, h, gu.shape[1] // 2, (S["sgu"].shape[0] // 2
+                                                      if case.get("shared", True) else 0)
+    held = lambda n: pkg.lib().i4_dmoe_workspace_bytes_h(n, *sizes)
+    slots = lambda n: min(n, 1024) * top_k * h * 4
+    assert held(T) > slots(T) and held(8) < slots(8) + 8 * 2 * sizes[0] + 8 * 4096 * top_k
     got = call(0, T)
-    assert torch.isfinite(got[0].float()).all()
+    if case.get("nonfinite"):
+        bad = [t for t in range(T) if not torch.isfinite(got[0][t].float()).all()]
+        assert bad == [3, 9, 17]
+    else:
+        assert torch.isfinite(got[0].float()).all()
     if case.get("skew"):
         assert (got[1] == 3).sum() == T
     for a in range(0, T, 8):
         if T > 200 and 16 <= a < T - 24 and a % 128:
             continue
         for u, v in zip(got, call(a, min(a + 8, T))):
-            assert torch.equal(u[a:a + 8], v), f"tokens {a}.. of {T}"
+            u = u[a:a + 8]
+            assert torch.equal(torch.isnan(u), torch.isnan(v)), f"tokens {a}.. of {T}"
+            assert torch.equal(torch.nan_to_num(u), torch.nan_to_num(v)), f"tokens {a}.. of {T}"
