@@ -679,15 +679,28 @@ int linear_ksplit(int M, int N, int K) {
 }
 
 // Whether a dense linear launch takes the 128-row tiles: a round of 256 of them (one
-// workgroup per CU) takes the same time full or not, so they have to fill their rounds.
-// us, 64-row tiles / 128-row tiles at K 2048: bf16 groups of 32 at 112 tiles 44 / 50, 140
-// 67 / 52, 240 85 / 57, 320 119 / 100, 640 207 / 156; fp16 groups of 128 at 192 tiles
-// 40 / 41, 240 49 / 45, 320 63 / 77, 512 93 / 80, 640 113 / 117.
-static bool linear_big(int xt, int M, int N) {
+// workgroup per CU) takes the same time full or not, so they have to fill their rounds, the
+// more the less they gain on the 64-row kernel.  Measured over K 128..8192, N 512..8192,
+// 300..9000 rows, groups of 32, 64, 128 and 256, time of the 128-row tiles over that of the
+// 64-row ones (us at K 2048 where given):
+//   bf16, groups under 128: 0.45-0.93 from half a round on (140 tiles 67 -> 52, 320 119 ->
+//     100, 640 207 -> 156).
+//   bf16, longer groups (one correction a superchunk): 0.7-0.9 in one or three and more
+//     rounds, but two rounds filled to 0.55-0.7 take 0.95-1.10, from three quarters 0.7-1.0.
+//   fp16 (scales folded into B, the 64-row kernel's work per MFMA is smaller): nine tenths
+//     filled.  Groups under 128: one round 0.70-0.93 at every K, two 0.8-1.0 from K 512,
+//     more 0.8-1.0 at K from 1536 and at multiples of 512, 1.0-1.15 at the others.  Longer
+//     groups: one round 0.8-1.0 from K 512 (256 tiles 51 -> 46; 384 1.04), more 0.86-0.97
+//     from K 2048 (512 tiles 91 -> 83) and up to 1.3 below.
+static bool linear_big(int xt, int M, int N, int K, bool long_groups) {
   if (N % (32 * TG_NW) != 0) return false;
   const int64_t tiles = (int64_t)(N / (32 * TG_NW)) * ((M + TG_TOK - 1) / TG_TOK);
-  const int64_t slots = (tiles + 255) / 256 * 256;
-  return xt == I4_BF16 ? 2 * tiles > slots : 10 * tiles >= 9 * slots;
+  const int64_t rounds = (tiles + 255) / 256, slots = 256 * rounds;
+  if (xt == I4_BF16)
+    return long_groups && rounds == 2 ? 4 * tiles >= 3 * slots : 2 * tiles > slots;
+  if (10 * tiles < 9 * slots) return false;
+  if (long_groups) return K >= (rounds == 1 ? 512 : 2048);
+  return rounds == 1 || (rounds == 2 && K >= 512) || K >= 1536 || K % 512 == 0;
 }
 
 size_t linear_tile_workspace_bytes(int M, int N, int K) {
@@ -705,7 +718,8 @@ int launch_mfma_linear(const void* x, int M, const TW& w, const void* bias, void
     return I4_ERR_SHAPE;
   constexpr int COLS = 64 * MF_NB, TOK = LIN_TOK;
   if (w.N % COLS != 0 || w.K % 128 != 0 || w.E != 1) return I4_ERR_SHAPE;
-  if (linear_big(XT, M, w.N)) return launch_tile_gemm_linear<XT, ST>(x, M, w, bias, y, ot, s);
+  if (linear_big(XT, M, w.N, w.K, w.gshift >= 2))
+    return launch_tile_gemm_linear<XT, ST>(x, M, w, bias, y, ot, s);
   const int ks = linear_ksplit(M, w.N, w.K);
   if (ks > 1 && (!ws || ws_bytes < linear_tile_workspace_bytes(M, w.N, w.K)))
     return I4_ERR_WORKSPACE;

@@ -486,10 +486,11 @@ BIG_FMTS = ["ct-g32-bf16", "awq-g32-bf16", "awq-g128-bf16", "awq-g128-f16", "ct-
 
 
 @pytest.mark.parametrize("fmt", BIG_FMTS)
-@pytest.mark.parametrize("M,K", [(2048, 128), (1921, 384)])
+@pytest.mark.parametrize("M,K", [(2048, 128), (1921, 384), (2048, 512), (1921, 640)])
 def test_linear_128_row_tiles(pkg, dev, fmt, M, K):
-    """Enough rows for the 128 x 256 tiles (2048 -> 4096 outputs: 256 of them), a ragged last
-    tile of one row and an odd number of superchunks, against the oracle's float64 matmul."""
+    """Enough rows for the 128 x 256 tiles (2048 -> 4096 outputs: 256 of them; fp16 in groups of
+    128 takes them from K 512), a ragged last tile of one row and an odd number of
+    superchunks, against the oracle's float64 matmul."""
     rng = np.random.default_rng(M + K)
     w, dq, xdt = _ct_or_awq(pkg, dev, rng, 1, 4096, K, fmt)
     x = make_x(rng, (M, K), xdt)
