@@ -349,9 +349,12 @@ MoeWs carve(void* base, int T, int H, int I, int E, int topk, int tc) {
 
 // Tokens per pass: the 128-token tiles' passes need a workspace of their own size, so a
 // smaller one (the library's static scratch, one that a caller sized for 1024 tokens) is
-// served in passes of TCHUNK as any call of 1024 tokens is.
-int tokens_per_pass(int T, int H, int I, int E, int topk, size_t bytes) {
-  return T > TCHUNK && tile_gemm_fits(H, I, E, topk) &&
+// served in passes of TCHUNK as any call of 1024 tokens is.  So is a call of 1025 in fp16: its
+// second pass is one token's, and fp16 gains least from the large tiles (8 experts, top-2, H
+// 4096, I 1792, us in passes of TCHUNK / in one: 1025 tokens 209 / 244, 1026 247 / 251, 1100
+// 245 / 229; bf16 353 / 274 at 1025).
+int tokens_per_pass(int xt, int T, int H, int I, int E, int topk, size_t bytes) {
+  return T > TCHUNK + (xt == I4_F16) && tile_gemm_fits(H, I, E, topk) &&
                  carve(nullptr, T, H, I, E, topk, BIG_CHUNK).bytes <= bytes
              ? BIG_CHUNK
              : TCHUNK;
@@ -625,7 +628,7 @@ int moe_forward_impl(const void* x, int x_dtype, int T, const i4_moe_weights* we
   if (((uintptr_t)x & 15) || ((uintptr_t)out & 15) || ((uintptr_t)residual & 15))
     return I4_ERR_ALIGN;
   const int H = gu.K, I = dn.K, E = gu.E;
-  const int tc = tokens_per_pass(T, H, I, E, topk, workspace_bytes);
+  const int tc = tokens_per_pass(x_dtype, T, H, I, E, topk, workspace_bytes);
   MoeWs ws = carve(workspace, T, H, I, E, topk, tc);
   if (!workspace || workspace_bytes < ws.bytes) return I4_ERR_WORKSPACE;
   if ((uintptr_t)workspace & 255) return I4_ERR_ALIGN;
@@ -814,7 +817,8 @@ extern "C" {
 
 size_t i4_moe_workspace_bytes(int T, int H, int I, int E, int topk) {
   if (T < 1 || H < 1 || I < 1 || E < 1 || topk < 1) return 0;
-  return carve(nullptr, T, H, I, E, topk, tokens_per_pass(T, H, I, E, topk, SIZE_MAX)).bytes;
+  const int tc = tokens_per_pass(I4_BF16, T, H, I, E, topk, SIZE_MAX);  // either type
+  return carve(nullptr, T, H, I, E, topk, tc).bytes;
 }
 
 size_t i4_moe_status_offset(int T, int H, int I, int E, int topk) {

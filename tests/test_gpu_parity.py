@@ -499,7 +499,7 @@ def test_linear_128_row_tiles(pkg, dev, fmt, M, K):
 
 
 @pytest.mark.parametrize("fmt", BIG_FMTS)
-@pytest.mark.parametrize("T", [1025, 4100])
+@pytest.mark.parametrize("T", [1026, 4100])
 def test_moe_128_token_tiles(pkg, dev, fmt, T):
     """Calls of more than 1024 tokens run on 128-token tiles in passes of 4096: experts with 0,
     1, 16, 17, 33, 65, 128, 129 and 257 tokens in a pass, and a last pass of four tokens."""
