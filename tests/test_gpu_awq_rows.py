@@ -13,7 +13,9 @@ from tests import _gen
 from tests.test_gpu_parity import f_, host, make_x, t_
 
 pytestmark = pytest.mark.gpu
-DT = {"f16": torch.float16, "bf16": torch.bfloat16}
+# the output's rounding (half an ulp: 2^-11 / 2^-8 of a value) against the largest value,
+# with the fp32 sums' own error far below it
+TOL = {"f16": 1e-3, "bf16": 4e-3}
 CODE = {"f16": 1, "bf16": 2}
 
 
@@ -78,3 +80,62 @@ def test_two_streams_share_one_module(pkg, dev):
     for i in range(2):
         for n, y in enumerate(got[i]):
             assert torch.equal(y, want[i][n % 4])
+
+
+@pytest.mark.parametrize("xdt,G,zeros", [("f16", 128, True), ("bf16", 128, True),
+                                         ("bf16", 64, False), ("f16", 32, False)])
+@pytest.mark.parametrize("N,K", [(512, 2048), (1024, 2048), (2048, 1024), (768, 4096)])
+def test_few_rows_on_either_path(pkg, dev, xdt, G, zeros, N, K):
+    """3..8 rows, on both sides of the line between the GEMV and MFMA, with and without zero
+    points, K ranges that end inside a group: against float64, and by which memory of the
+    caller's workspace a call writes (MFMA: every fp32 partial behind the GEMV's pairs, and
+    not the status word; the GEMV: none of them)."""
+    lb = pkg.lib()
+    rng = np.random.default_rng(N + G)
+    w, dq = awq(pkg, dev, rng, N, K, G, xdt, zeros)
+    cw = w.c()
+    size = lambda M: lb.i4_linear_workspace_bytes(ctypes.byref(cw), M)
+    bias = t_(make_x(rng, (N,), xdt), dev)
+    took = set()
+    for M in (3, 4, 5, 6, 7, 8):
+        x = t_(make_x(rng, (M, K), xdt), dev)
+        mm = bool(lb.i4_linear_awq_mfma(ctypes.byref(cw), M))
+        took.add(mm)
+        nbytes = max(size(M), 256)
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+        head = max([256] + [lb.i4_dq_gemv_workspace_bytes(ctypes.byref(cw), r)
+                            for r in range(1, 9) if not lb.i4_linear_awq_mfma(
+                                ctypes.byref(cw), r)])
+        if mm:
+            assert (nbytes - head) % (M * N * 4) == 0 and nbytes > head
+            ws[head:].view(torch.int32).fill_(0x7FC0DEAD)  # a NaN no sum produces
+        y = torch.empty(M, N, dtype=x.dtype, device=dev)
+        rc = lb.i4_linear(x.data_ptr(), CODE[xdt], M, ctypes.byref(cw), bias.data_ptr(),
+                          y.data_ptr(), CODE[xdt], ws.data_ptr() if nbytes else None, nbytes,
+                          torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        ref = x.double().cpu().numpy() @ dq.T + bias.double().cpu().numpy()
+        assert i4ref.rel_err(y.double().cpu().numpy(), ref) <= TOL[xdt]
+        assert int(ws[:4].view(torch.int32)[0]) == 0
+        if mm:
+            assert not bool((ws[head:].view(torch.int32) == 0x7FC0DEAD).any())
+            assert not bool(ws[4:head].any())
+    assert False in took  # 3 rows: the GEMV
+
+
+@pytest.mark.parametrize("xdt", ["f16", "bf16"])
+def test_nonfinite_rows_stay_apart(pkg, dev, xdt):
+    """Infinities and NaN in some rows of x reach those rows' outputs only."""
+    rng = np.random.default_rng(79)
+    w, _ = awq(pkg, dev, rng, 2048, 4096, 128, xdt)
+    x = t_(make_x(rng, (37, 4096), xdt), dev)
+    clean = pkg.ops.linear(x, w)
+    bad = {0: float("inf"), 15: float("nan"), 16: float("-inf"), 36: float("nan")}
+    for r, v in bad.items():
+        x[r, 37 * r % 4096] = v
+    got = pkg.ops.linear(x, w)
+    for r in range(37):
+        if r in bad:
+            assert not bool(torch.isfinite(got[r]).any())
+        else:
+            assert torch.equal(got[r], clean[r])

@@ -524,6 +524,34 @@ def test_moe_128_token_tiles(pkg, dev, fmt, T):
     _check_moe(pkg, moe, dgu, ddn, x, xdt, dev, logits=lg, residual=x)
 
 
+@pytest.mark.parametrize("fmt", ["ct-g32-bf16", "awq-g128-f16"])
+def test_nonfinite_rows_stay_apart_on_large_tiles(pkg, dev, fmt):
+    """Infinities and NaN in some rows of x (or some tokens) reach those rows only: the dense
+    128-row tiles, and the MoE block in one pass of 128-token tiles with its grouping,
+    router and combine (logits given, so that the routing stays)."""
+    rng = np.random.default_rng(83)
+    bad = {0: float("inf"), 127: float("nan"), 128: float("-inf"), 999: float("nan")}
+    w, _, xdt = _ct_or_awq(pkg, dev, rng, 1, 8192, 512, fmt)
+    tile = w.to_tile()
+    x = t_(make_x(rng, (1100, 512), xdt), dev)  # 1000 rows: 32 x 8 tiles, a whole round
+    E, H, I, k = 24, 512, 128, 4
+    gu, _, _ = _ct_or_awq(pkg, dev, rng, E, 2 * I, H, fmt)
+    dn, _, _ = _ct_or_awq(pkg, dev, rng, E, H, I, fmt)
+    moe = pkg.FusedPackedMoE.from_stacked(gu, dn, torch.zeros(E, H, dtype=x.dtype, device=dev),
+                                          top_k=k)
+    lg = t_(make_x(rng, (1100, E), xdt), dev)
+    run = lambda v: (pkg.ops.linear(v[:1000], tile),
+                     pkg.moe_forward(v, moe.gate_up, moe.down, k, logits=lg, residual=v,
+                                     gate_up_tile=moe.gate_up_tile, down_tile=moe.down_tile))
+    clean = run(x)
+    for r, v in bad.items():
+        x[r, 3 * r % 512] = v
+    for got, ref in zip(run(x), clean):
+        rows = torch.tensor([r for r in range(len(ref)) if r not in bad], device=dev)
+        assert torch.isfinite(ref).all() and torch.equal(got[rows], ref[rows])
+        assert not torch.isfinite(got[list(bad)]).all(dim=1).any()
+
+
 def test_packed_qkv_matches_three_linears(pkg, dev):
     """q, k, v in one launch equal the three separate launches bit for bit (each row's dot
     product does not depend on its neighbours): AWQ parts, and CT parts with and without
