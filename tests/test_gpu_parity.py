@@ -463,6 +463,7 @@ def test_linear_awq_rows(pkg, dev, M, N, K, xdt, sdt, G):
     y = torch.empty_like(got)
     cw, xd, bd = w.c(), t_(x, dev), t_(bias, dev)
     lb = pkg.lib()
+    assert lb.i4_linear_awq_mfma(ctypes.byref(cw), M)
     code = {"f16": 1, "bf16": 2}[xdt]
     assert lb.i4_linear(xd.data_ptr(), code, M, ctypes.byref(cw), bd.data_ptr(), y.data_ptr(),
                         code, None, 0, torch.cuda.current_stream().cuda_stream) == 0
