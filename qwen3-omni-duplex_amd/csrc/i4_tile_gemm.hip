@@ -8,12 +8,14 @@
 // entry; the 128 activation rows of a superchunk are staged once for all eight waves, double
 // buffered, loaded one superchunk ahead.  One workgroup fills a CU (up to 256 VGPRs).
 //
-// Bound: issue.  A superchunk takes 2.9 us with groups of 32 (4 FMAs per MFMA apply the
-// scales: MFMA busy 29 %, VALU 51 %, LDS 37 % of the cycles, the two waves of a SIMD
-// overlapping little) and 2.3 us with folded scales, the same on an idle card.  Measured:
-// bf16 2048 -> 5120, 1500 rows 109 -> 50 us (630 TFLOP/s); the 3001-token MoE block 939 ->
-// 597 us.  Slower: waves in a 2 x 4 arrangement of 64 x 64 (54 us), 128 x 128 tiles of four
-// waves, two workgroups per CU (62 us), MFMA and FMA groups interleaved by hand (58-62 us).
+// Bound: issue.  A superchunk takes 2.9 us with groups of 32 (5.9 vector instructions per
+// MFMA, 4 of them FMAs that apply the scales: MFMA busy 29 %, VALU 51 %, LDS 41 % of the
+// cycles, the two waves of a SIMD overlapping little) and 2.3 us with folded scales (2.6;
+// MFMA 37 %), the same on an idle card.  Measured: bf16 2048 -> 5120, 1500 rows 109 -> 50 us
+// (630 TFLOP/s); the 3001-token MoE block, with its router and combine, 942 -> 523 us.
+// Slower: waves in a 2 x 4 arrangement of 64 x 64 (54 us), 128 x 128 tiles of four waves, two
+// workgroups per CU (62 us), MFMA and FMA groups interleaved by hand (58-62 us), a branch
+// around the last step of an odd superchunk count, whose products alone are skipped (245 us).
 // The zero points' presence is a template argument for bf16: chosen at run time, the
 // compiler multiplied and selected in every group (72 us).
 #include "i4_tile_mfma.h"
