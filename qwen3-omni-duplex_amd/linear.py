@@ -6,7 +6,7 @@ E = 1 case of the expert gather.  The reference launches one kernel per row of
 x (:154-155); here all rows go in one launch, and q/k/v can share one launch
 (PackedQKV, patch_attention(fuse_qkv=True)).  Batches of TILE_ROWS rows or more
 (prefill) run on MFMA from a tile-layout copy of the weight, which streams each
-weight tile once per 64 rows instead of once per row.
+weight tile once per 64 or 128 rows instead of once per row.
 """
 from __future__ import annotations
 
@@ -57,13 +57,15 @@ class PackedLinear(nn.Module):
         self.register_buffer("scale", w.scale, persistent=False)
         self.register_buffer("zeros", w.zeros, persistent=False)
         self.register_buffer("bias", bias, persistent=False)
-        self.workspace = ops.Workspace()  # this module's split-K workspace, kept across calls
+        # the split-K workspace of calls of a few rows (and of the tile copy), kept across
+        # calls; several rows on AWQ in place allocate their partials per call
+        self.workspace = ops.Workspace()
 
     @classmethod
     def from_qweight(cls, w: QWeight, bias: torch.Tensor | None = None,
                      repack: bool = True, tile: bool = True) -> "PackedLinear":
         """From a CT or AWQ weight; AWQ is repacked to CT+zeros unless repack=False
-        (the in-place AWQ GEMV, which keeps no tile copy)."""
+        (AWQ in place: the GEMV for a few rows, MFMA for several; no tile copy)."""
         m = cls()
         m._install(w.to_ct() if repack else w, bias, tile)
         return m
@@ -108,7 +110,7 @@ def concat_rows(parts: list[QWeight]) -> QWeight:
 def concat_cols_awq(parts: list[QWeight]) -> QWeight:
     """One AWQ weight (E = 1) holding the output columns of parts in order, still in
     AutoAWQ packing ([K][N / 8] words, [groups][N] scales, [groups][N / 8] zero words):
-    the in-place GEMV then serves q, k and v in one launch.  A part without zero
+    one in-place call then serves q, k and v.  A part without zero
     points gets explicit 8s when another has them."""
     p0 = parts[0]
     for p in parts:
@@ -147,8 +149,8 @@ class PackedQKV(nn.Module):
     @classmethod
     def from_qweights(cls, q: QWeight, k: QWeight, v: QWeight, biases=None,
                       repack: bool = True) -> "PackedQKV":
-        """repack=False keeps AWQ parts in AWQ packing (concat_cols_awq, the in-place
-        GEMV, no tile copy); otherwise the rows are concatenated in CT (concat_rows)."""
+        """repack=False keeps AWQ parts in AWQ packing (concat_cols_awq, read in place,
+        no tile copy); otherwise the rows are concatenated in CT (concat_rows)."""
         in_place = not repack and all(p.layout == "awq" for p in (q, k, v))
         w = concat_cols_awq([q, k, v]) if in_place else concat_rows([q, k, v])
         bias = None
