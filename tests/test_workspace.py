@@ -13,7 +13,7 @@ CPU = torch.device("cpu")
 def ops(pkg, monkeypatch):
     monkeypatch.setattr(pkg.ops, "_capturing", lambda device: pkg.ops._test_capture,
                         raising=False)
-    pkg.ops._test_capture = False
+    monkeypatch.setattr(pkg.ops, "_test_capture", False, raising=False)
     return pkg.ops
 
 
